@@ -878,7 +878,7 @@ void launch_mg0_smooth(const Geo& g, const MgTab& wd0, int src, bool rz, const d
 template <int CPL = 1>
 static Tile3Grid mg_tile_grid(const Geo& g)
 {
-    Tile3Grid t = tile3_grid<CPL>(g);
+    Tile3Grid t = tile3_grid_deep<CPL>(g);
     t.kz += t.kz & 1;
     while (t.kz > 2 && t.tiles_x * t.tiles_y * ((g.n[2] + t.kz - 1) / t.kz) * kTileBlock <
                            512 * 256)

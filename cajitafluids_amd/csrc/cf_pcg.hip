@@ -1268,7 +1268,11 @@ void launch_pcg_xfix(const Geo& g, T* x, const T* p, const PcgState* st, hipStre
 
 int reduction_blocks_max(const Geo& g)
 {
-    const int t = g.dim == 3 ? tile3_blocks<1>(g) : 0; // the largest tile grid
+    // the largest tile grid (up to 64 cells along x, FP32 pairs have as many
+    // tiles and chunks half as deep)
+    const int t1 = g.dim == 3 ? tile3_blocks<1>(g) : 0;
+    const int t2 = g.dim == 3 ? tile3_blocks<2>(g) : 0;
+    const int t = t1 > t2 ? t1 : t2;
     return t > kRedBlocks ? t : kRedBlocks;
 }
 

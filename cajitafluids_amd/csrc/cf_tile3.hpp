@@ -123,18 +123,56 @@ struct epi_loads_late<E, std::void_t<decltype(E::kLate)>> : std::bool_constant<E
 {
 };
 
+// z chunks of at least 16 planes (FP32 pairs: 8, as many blocks as the
+// one-cell-per-lane tiling): the grid of the multigrid tiles before they
+// shorten it, and of every kernel on the largest grids.
 template <int CPL>
-inline Tile3Grid tile3_grid(const Geo& g)
+inline Tile3Grid tile3_grid_deep(const Geo& g)
 {
     using namespace tile3;
     Tile3Grid t;
     t.tiles_x = (g.n[0] + tx<CPL>() - 1) / tx<CPL>();
     t.tiles_y = (g.n[1] + TY - 1) / TY;
-    // z chunks: as many blocks as the one-cell-per-lane tiling
     const int zc = 16 * CPL;
     t.kz = g.n[2] / zc > 16 / CPL ? g.n[2] / zc : 16 / CPL;
     t.nchunk = (g.n[2] + t.kz - 1) / t.kz;
     t.work = t.tiles_x * t.tiles_y * t.nchunk;
+    return t;
+}
+
+// The PCG tiles' grid.  A block marches its planes one after the other
+// (1.1 us a plane for a lone block, direction and update alike), so below
+// about 200^3 the depth of a chunk sets the time, and the blocks should
+// spread evenly over the 256 CUs.  The chunk depth is the one that minimises
+//   max(blocks per CU, 2) * (planes + 2):
+// the last CU's blocks times a block's loads (its planes and two halo
+// planes); the 2 because a lone block on a CU leaves its memory latency
+// bare.  A sweep over the depth picks the same one or one within 3% of it
+// (us per FP64 iteration, direction and update, 16-plane chunks before):
+// 45 x 52 x 61 55.0 -> 22.7, 128^3 57.2 -> 37.7, 160 x 144 x 180 74.8 ->
+// 59.3, 220^3 154.4 -> 138.1, 256^3 195.3 -> 192.6; FP32: 64^3 43.8 -> 25.3,
+// 220^3 85.9 -> 77.9.  Grids of 2048 deep blocks and more keep those (an
+// uneven last round is under an eighth of the work there), so no grid has
+// more blocks than the larger of the two (reduction_blocks_max).
+template <int CPL>
+inline Tile3Grid tile3_grid(const Geo& g)
+{
+    Tile3Grid t = tile3_grid_deep<CPL>(g);
+    if (t.work >= kRedBlocks)
+        return t;
+    const int tiles = t.tiles_x * t.tiles_y;
+    int64_t best = INT64_MAX;
+    for (int nc = 1; nc <= (g.n[2] + 1) / 2 && tiles * nc <= kRedBlocks; ++nc) {
+        const int kz = (g.n[2] + nc - 1) / nc;
+        const int per_cu = (tiles * nc + 255) / 256;
+        const int64_t cost = (int64_t)(per_cu > 2 ? per_cu : 2) * (kz + 2);
+        if (cost < best) {
+            best = cost;
+            t.kz = kz;
+        }
+    }
+    t.nchunk = (g.n[2] + t.kz - 1) / t.kz;
+    t.work = tiles * t.nchunk;
     return t;
 }
 
