@@ -74,6 +74,36 @@ struct MgParentMap
     int64_t base, sy, sz;
 };
 
+// A level's operator by the place of a cell along each axis (class 0 in
+// between, 1 first, 2 last, 3 both): diagonal and Jacobi weight at
+// cx + 4 cy + 16 cz, couplings along x at cy + 4 cz, along y at cx + 4 cz,
+// along z at cx + 4 cy.  A row outside the domain has class kMgOutside in place
+// of cx + 4 cy, a plane outside it class 4: entries of 0.
+constexpr int kMgOutside = 64;
+template <class T>
+struct MgOpTab
+{
+    T diag[2 * kMgOutside + 1], w[2 * kMgOutside + 1], cx[16], cy[16], cz[16];
+};
+struct MgOp
+{
+    MgOpTab<double> d;
+    MgOpTab<float> f; // the FP64 entries rounded
+};
+
+// One level's legs in a launch each (cf_mg_fused.hip): its cells and its
+// parents' storage, and the tiling.
+struct MgFused
+{
+    int dim, n[3], periodic[3];
+    int tiles_x, core_x, tiles_y, core_y, nchunk, kz, work;
+    double alpha;
+    double coupling; // of every pair of neighbours, or 0 if they differ
+    MgParentMap lv, pm;
+    // elements from a plane's first owned cell to its last, and plane strides
+    unsigned len, plen, lsz, psz;
+};
+
 // Source of the values a smoothing sweep reads:
 //   first:   x = w b (the sweep from zero, computed on the fly)
 //   plain:   x = xi
@@ -131,6 +161,24 @@ void launch_mg_smooth3_f32(const Geo& g, const Geo& gw, int src, bool rz, const 
 void launch_mg_resrestrict3_f32(const Geo& g, const float* x, const float* b, double* bc,
                                 float* bc32, MgParentMap pm, const PcgState* st, hipStream_t s,
                                 int cpl);
+
+// Whole legs of a level whose axes are all coarsened, with nu = 2 or 3 sweeps
+// (false otherwise); fills f but for the storage maps.  f32: the level runs in
+// FP32; coupling: a padded level's, 0 on a compact one.  Down: x = nu sweeps
+// from zero on b, bc the parents' right-hand side.  Up: xo = nu sweeps from
+// x + alpha xc; with rz also r.z = b . xo as above.  FP32 levels: as the FP32
+// sweeps below (r64: the rz leg's right-hand side).
+bool mg_fused_level(const MgLev& L, int nu, bool f32, double coupling, MgFused& f);
+void launch_mg_down(const MgFused& f, const MgOp* op, int nu, const double* b, double* x,
+                    double* bc, PcgState* st, RedBuf rb, hipStream_t s);
+void launch_mg_up(const MgFused& f, const MgOp* op, int nu, bool rz, const double* b,
+                  const double* x, const double* xc, double* xo, PcgState* st, RedBuf rb,
+                  hipStream_t s);
+void launch_mg_down_f32(const MgFused& f, const MgOp* op, int nu, const float* b, float* x,
+                        double* bc, float* bc32, PcgState* st, RedBuf rb, hipStream_t s);
+void launch_mg_up_f32(const MgFused& f, const MgOp* op, int nu, const float* b,
+                      const double* r64, const float* x, const double* xc, const float* xc32,
+                      float* xo, PcgState* st, RedBuf rb, hipStream_t s);
 
 // Compact levels.
 void launch_mg_first(const MgLev& L, const double* b, double* x, const PcgState* st,
@@ -194,6 +242,11 @@ class Multigrid
     std::vector<MgTab> _wt;  // level 0 and tiled levels: omega / diag by wall count
     std::vector<MgParentMap> _pm; // parent index of level l's cells in level l + 1
     std::vector<MgLev> _lev; // _lev[0]: level-0 dims and coarsening only
+    // levels whose legs run as one launch each (tiling; work 0: the others)
+    // [0]: in FP64, [1]: in FP32 (levels 0 and 1)
+    std::vector<MgFused> _fz[2];
+    bool fused(int l) const { return _fz[0][l].work > 0; }
+    MgOp op_table(int l) const;
     std::unique_ptr<Buffers> _buf;
 };
 

@@ -38,10 +38,13 @@ struct Multigrid::Buffers
     std::vector<std::unique_ptr<DevArray<double>>> vec;
     std::vector<double*> X, T, B, res;
     MgTail* tail = nullptr; // device copy
+    MgOp* op = nullptr;     // operator tables of the fused levels, device
     ~Buffers()
     {
         if (tail)
             (void)hipFree(tail);
+        if (op)
+            (void)hipFree(op);
     }
 };
 
@@ -204,8 +207,25 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
             B.vec.push_back(std::move(a));
         }
     }
+    for (int v = 0; v < 2; ++v) {
+        _fz[v].assign(nl, MgFused{});
+        for (int l = 0; l < _tail0 && l < last; ++l) {
+            MgFused& f = _fz[v][l];
+            const double c = l == 0 ? -g.s : (l < _nt ? -_lg[l].s : 0.0);
+            if (!mg_fused_level(_lev[l], _nu, v == 1, c, f))
+                continue;
+            f.lv = l == 0 ? MgParentMap{g.idx(g.h, g.h, g.own_lo(2)), g.px, g.px * g.py}
+                          : _pm[l - 1];
+            f.pm = _pm[l];
+            f.len = (unsigned)(f.lv.sy * (_lev[l].n[1] - 1) + _lev[l].n[0]);
+            f.plen = (unsigned)(_pm[l].sy * (_lev[l + 1].n[1] - 1) + _lev[l + 1].n[0]);
+            f.lsz = (unsigned)f.lv.sz;
+            f.psz = (unsigned)_pm[l].sz;
+        }
+    }
+    // a fused level's upward leg ends in T
     for (int l = 0; l < nl; ++l)
-        B.res[l] = (mg_level_swaps(l == last, _nu, _coarse) & 1) ? B.T[l] : B.X[l];
+        B.res[l] = fused(l) || (mg_level_swaps(l == last, _nu, _coarse) & 1) ? B.T[l] : B.X[l];
     if (last >= 1) {
         MgTail h{};
         h.l0 = _tail0;
@@ -227,10 +247,73 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
         B.tail = (MgTail*)p;
         CF_HIP(hipMemcpyAsync(B.tail, &h, sizeof(MgTail), hipMemcpyHostToDevice, s));
     }
+    std::vector<MgOp> op(nl);
+    for (int l = 0; l < nl; ++l)
+        if (fused(l))
+            op[l] = op_table(l);
+    {
+        void* p = nullptr;
+        CF_HIP(hipMalloc(&p, nl * sizeof(MgOp)));
+        B.op = (MgOp*)p;
+        CF_HIP(hipMemcpyAsync(B.op, op.data(), nl * sizeof(MgOp), hipMemcpyHostToDevice, s));
+    }
     CF_HIP(hipStreamSynchronize(s));
 }
 
 Multigrid::~Multigrid() = default;
+
+// The operator of level l by class (MgOpTab): the entries its sweep kernels
+// read from their tables (padded levels) or compute (compact ones).
+MgOp Multigrid::op_table(int l) const
+{
+    MgOp t{};
+    const MgLev& L = _lev[l];
+    const bool padded = l == 0 || l < _nt;
+    const Geo& lg = l < _nt ? _lg[l] : _g;
+    for (int id = 0; id < 64; ++id) {
+        const int cl[3] = {id & 3, (id >> 2) & 3, id >> 4};
+        int64_t e[3] = {1, 1, 1}, area[3], K = 0;
+        int walls = 0;
+        for (int d = 0; d < L.dim; ++d)
+            // only the last box along an axis may be cut short
+            e[d] = cl[d] & 2 ? L.n0[d] - ((int64_t)(L.n[d] - 1) << L.shift[d])
+                             : (int64_t)1 << L.shift[d];
+        for (int d = 0; d < 3; ++d)
+            area[d] = e[0] * e[1] * e[2] / e[d];
+        for (int d = 0; d < L.dim; ++d) {
+            const bool lo = !L.periodic[d] && (cl[d] & 1) && L.solid[d][0];
+            const bool hi = !L.periodic[d] && (cl[d] & 2) && L.solid[d][1];
+            walls += lo + hi;
+            K += (lo ? 0 : area[d]) + (hi ? 0 : area[d]);
+        }
+        if (padded) {
+            t.d.diag[id] = lg.diag[walls];
+            t.d.w[id] = _wt[l].v[walls];
+        } else {
+            t.d.diag[id] = (double)K * L.s;
+            t.d.w[id] = K > 0 ? L.omega / t.d.diag[id] : 0.0;
+        }
+        const double c[3] = {padded ? -lg.s : -((double)area[0] * L.s),
+                             padded ? -lg.s : -((double)area[1] * L.s),
+                             padded ? -lg.s : -((double)area[2] * L.s)};
+        if (cl[0] == 0)
+            t.d.cx[cl[1] + 4 * cl[2]] = c[0];
+        if (cl[1] == 0)
+            t.d.cy[cl[0] + 4 * cl[2]] = c[1];
+        if (cl[2] == 0)
+            t.d.cz[cl[0] + 4 * cl[1]] = c[2];
+    }
+    for (int id = 0; id < 64; ++id) {
+        t.f.diag[id] = (float)t.d.diag[id];
+        t.f.w[id] = (float)t.d.w[id];
+    }
+    for (int id = 0; id < 16; ++id) {
+        t.f.cx[id] = (float)t.d.cx[id];
+        t.f.cy[id] = (float)t.d.cy[id];
+        t.f.cz[id] = (float)t.d.cz[id];
+    }
+    return t;
+}
 
 // x = w b on level l
 void Multigrid::first(int l, const double* b, double* x, PcgState* st)
@@ -352,18 +435,27 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
         float* b0 = B.f[2].ptr;
         if (!b32_ready)
             launch_mg_cast32(_g, r, b0, st, _s);
-        if (_nu == 1)
-            launch_mg0_first_f32(_g, _wt[0], b0, x, st, _s);
-        else
-            smooth32(0, MG_FIRST, false, nullptr, b0, r, x, nullptr, st, rb);
-        for (int it = 2; it < _nu; ++it) {
-            smooth32(0, MG_PLAIN, false, x, b0, r, t, nullptr, st, rb);
-            std::swap(x, t);
+        if (fused(0)) {
+            launch_mg_down_f32(_fz[1][0], B.op, _nu, b0, x, B.B[1], f1 ? B.f1[2].ptr : nullptr, st,
+                               rb, _s);
+        } else {
+            if (_nu == 1)
+                launch_mg0_first_f32(_g, _wt[0], b0, x, st, _s);
+            else
+                smooth32(0, MG_FIRST, false, nullptr, b0, r, x, nullptr, st, rb);
+            for (int it = 2; it < _nu; ++it) {
+                smooth32(0, MG_PLAIN, false, x, b0, r, t, nullptr, st, rb);
+                std::swap(x, t);
+            }
+            launch_mg_resrestrict3_f32(_lg[0], x, b0, B.B[1], f1 ? B.f1[2].ptr : nullptr, _pm[0],
+                                       st, _s, 2);
         }
-        launch_mg_resrestrict3_f32(_lg[0], x, b0, B.B[1], f1 ? B.f1[2].ptr : nullptr, _pm[0], st,
-                                   _s, 2);
         x32 = x;
-        if (f1) {
+        if (f1 && fused(1)) {
+            x1f = B.f1[0].ptr;
+            launch_mg_down_f32(_fz[1][1], B.op + 1, _nu, B.f1[2].ptr, x1f, B.B[2], nullptr, st, rb,
+                               _s);
+        } else if (f1) {
             float *y = B.f1[0].ptr, *u = B.f1[1].ptr;
             const float* b1 = B.f1[2].ptr;
             if (_nu == 1)
@@ -383,6 +475,10 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
         const double* b = l == 0 ? r : B.B[l];
         double* x = B.X[l];
         double* t = B.T[l];
+        if (fused(l)) {
+            launch_mg_down(_fz[0][l], B.op + l, _nu, b, x, B.B[l + 1], st, rb, _s);
+            continue;
+        }
         if (_nu == 1)
             first(l, b, x, st);
         else
@@ -400,6 +496,11 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
     double* x = nullptr;
     for (int l = _tail0 - 1; l >= l0; --l) {
         const double* b = l == 0 ? r : B.B[l];
+        if (fused(l)) {
+            x = B.T[l];
+            launch_mg_up(_fz[0][l], B.op + l, _nu, l == 0, b, B.X[l], B.res[l + 1], x, st, rb, _s);
+            continue;
+        }
         x = pre_odd ? B.T[l] : B.X[l];
         double* t = pre_odd ? B.X[l] : B.T[l];
         smooth(l, MG_PROLONG, l == 0 && _nu == 1, x, b, t, st, rb);
@@ -415,11 +516,17 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
             float* y = x1f;
             float* u = y == B.f1[0].ptr ? B.f1[1].ptr : B.f1[0].ptr;
             const float* b1 = B.f1[2].ptr;
-            smooth32(1, MG_PROLONG, false, y, b1, nullptr, u, nullptr, st, rb);
-            std::swap(y, u);
-            for (int it = 1; it < _nu; ++it) {
-                smooth32(1, MG_PLAIN, false, y, b1, nullptr, u, nullptr, st, rb);
+            if (fused(1)) {
+                launch_mg_up_f32(_fz[1][1], B.op + 1, _nu, b1, nullptr, y, B.res[2], nullptr, u, st,
+                                 rb, _s);
                 std::swap(y, u);
+            } else {
+                smooth32(1, MG_PROLONG, false, y, b1, nullptr, u, nullptr, st, rb);
+                std::swap(y, u);
+                for (int it = 1; it < _nu; ++it) {
+                    smooth32(1, MG_PLAIN, false, y, b1, nullptr, u, nullptr, st, rb);
+                    std::swap(y, u);
+                }
             }
             xc32 = y;
         }
@@ -428,6 +535,11 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
         float* xf = x32;
         float* tf = xf == B.f[0].ptr ? B.f[1].ptr : B.f[0].ptr;
         const float* b0 = B.f[2].ptr;
+        if (fused(0)) {
+            launch_mg_up_f32(_fz[1][0], B.op, _nu, nullptr, r, xf, xc32 ? nullptr : B.res[1], xc32,
+                             tf, st, rb, _s);
+            return tf;
+        }
         smooth32(0, MG_PROLONG, _nu == 1, xf, b0, r, tf, xc32, st, rb);
         std::swap(xf, tf);
         for (int it = 1; it < _nu; ++it) {
