@@ -672,12 +672,89 @@ __device__ __forceinline__ void mg_coarsest_wave(const MgLev& L, const double* _
 }
 
 // ---- the small levels in one workgroup ------------------------------------------------
-// Same cycle as the host runs on the large levels (Multigrid::vcycle), one
-// phase per sweep, __syncthreads between phases.  Every vector of these
-// levels lives in LDS (level l: X, T, B of ncell each from element
-// T->off[l]); the kernel reads level l0's right-hand side from global memory
-// and writes its cycle result to T->res[l0].
-#define CF_BLOCK_STRIDE(id, count) for (int id = threadIdx.x; id < (count); id += blockDim.x)
+// The cycle of the coarsest levels, every vector in LDS (level l: X, T, B of
+// ncell each from element T->off[l]).  A thread keeps its cells of a level
+// (id = thread + kMgTailThreads c) through all its sweeps: operator entries
+// (from the level's class tables), b, x and the LDS places of the neighbours
+// in registers, so a sweep is six LDS reads, its arithmetic and one write,
+// and one barrier.  Levels of at most one wave's cells run in wave 0 without
+// barriers.  A neighbour across a wall is read from a slot of -0: the
+// couplings are negative, so it adds +0, the term fma(0, 0, y) of the
+// grid kernels.  What bounds it is that chain: about 50 dependent phases of
+// 0.3 us.  256^3 (levels of 16^3 and below): 24 us; with every cell's entries
+// computed in every sweep (an FP64 division, integer face counts), a parent's
+// eight residuals in one thread and 8^3 as the largest level it took 35.
+// 391 x 263 (49 x 33 and below): 56 -> 19; 190 x 182 x 149: 58 -> 19.
+struct TailCell
+{
+    double diag, w, cx, cy, cz, b, x;
+    // the neighbours' elements of the level's vector, -x +x, -y +y, -z +z, in
+    // 13 bits each and counted from the slot of -0 ahead of it
+    int nb[3];
+};
+
+// The cell's operator entries and neighbours from its MgTailInfo.
+__device__ __forceinline__ void tail_cell(const MgOpTab<double>* op, const MgTailInfo& f,
+                                          TailCell& t)
+{
+    const int cls = (int)((unsigned)f.x >> 26);
+    t.diag = op->diag[cls];
+    t.w = op->w[cls];
+    t.cx = op->cx[cls >> 2];
+    t.cy = op->cy[(cls & 3) + ((cls >> 4) << 2)];
+    t.cz = op->cz[cls & 15];
+    t.nb[0] = f.x;
+    t.nb[1] = f.y;
+    t.nb[2] = f.z;
+}
+
+// The sum of a cell's children's residuals r of the level above (n0 cells
+// along x, n01 in a plane), z, y, x order.
+__device__ __forceinline__ double tail_children(const MgTailInfo& f, const double* r, int n0,
+                                                int n01)
+{
+    const int base = (int)((unsigned)f.w >> 16), has = (f.y >> 26) & 7;
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const bool in = (q & has) == q;
+        v[q] = r[in ? base + (q & 1) + (q & 2 ? n0 : 0) + (q & 4 ? n01 : 0) : base];
+    }
+    double sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        sum = (q & has) == q ? sum + v[q] : sum;
+    return sum;
+}
+
+// y = A x at the cell, x the level's vector in LDS
+__device__ __forceinline__ double tail_apply(const TailCell& t, int dim, const double* x)
+{
+    double y = t.diag * t.x;
+    const double* z = x - 1; // the slot of -0
+    y = fma(t.cx, z[t.nb[0] & 0x1fff], y);
+    y = fma(t.cx, z[(t.nb[0] >> 13) & 0x1fff], y);
+    y = fma(t.cy, z[t.nb[1] & 0x1fff], y);
+    y = fma(t.cy, z[(t.nb[1] >> 13) & 0x1fff], y);
+    if (dim == 3) {
+        y = fma(t.cz, z[t.nb[2] & 0x1fff], y);
+        y = fma(t.cz, z[(t.nb[2] >> 13) & 0x1fff], y);
+    }
+    return y;
+}
+
+// Calls f(cell, id) for the thread's cells of a level of n cells.
+template <class F>
+__device__ __forceinline__ void tail_each(int n, TailCell (&t)[kMgTailCells], F&& f)
+{
+#pragma unroll
+    for (int c = 0; c < kMgTailCells; ++c)
+        if (c * kMgTailThreads < n) {
+            const int id = (int)threadIdx.x + c * kMgTailThreads;
+            if (id < n)
+                f(t[c], id);
+        }
+}
 
 __global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(const MgTail* __restrict__ T,
                                                             const PcgState* st)
@@ -686,75 +763,151 @@ __global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(const MgTail* __rest
     if (st->done)
         return;
     const int l0 = T->l0, last = T->last, nu = T->nu, coarse = T->coarse;
-    auto X = [&](int l) { return lds + T->off[l]; };
-    auto Tv = [&](int l) { return lds + T->off[l] + T->lev[l].ncell; };
-    auto Bv = [&](int l) { return lds + T->off[l] + 2 * T->lev[l].ncell; };
-    auto res = [&](int l) { return (mg_level_swaps(l == last, nu, coarse) & 1) ? Tv(l) : X(l); };
+    const int dim = T->lev[l0].dim;
+    const double alpha = T->lev[l0].alpha;
+    // the vectors of level l: X and T with their slot of -0 ahead, and B
+    auto X = [&](int l) { return lds + T->off[l] + 1; };
+    auto Tv = [&](int l) { return lds + T->off[l] + 2 + T->lev[l].ncell; };
+    auto Bv = [&](int l) { return lds + T->off[l] + 2 + 2 * T->lev[l].ncell; };
+    MgOpTab<double>* ops = reinterpret_cast<MgOpTab<double>*>(lds + T->off[last + 1]);
+    // the cells' MgTailInfo: level l0's in memory, the others' copied to LDS
+    MgTailInfo* infos = reinterpret_cast<MgTailInfo*>(ops + (last - l0));
+    const int n_top = T->lev[l0].ncell, n_all = T->info_at[last + 1];
+    auto info = [&](int l, int id) -> MgTailInfo {
+        return l == l0 ? T->info[id] : infos[T->info_at[l] - n_top + id];
+    };
     {
+        for (int q = threadIdx.x; q < n_all - n_top; q += kMgTailThreads)
+            infos[q] = T->info[n_top + q];
+        constexpr int W = sizeof(MgOpTab<double>) / sizeof(double);
+        for (int q = threadIdx.x; q < (last - l0) * W; q += kMgTailThreads)
+            reinterpret_cast<double*>(ops)[q] =
+                reinterpret_cast<const double*>(&T->op[l0 + q / W].d)[q % W];
+        if ((int)threadIdx.x < last - l0) {
+            X(l0 + threadIdx.x)[-1] = -0.0;
+            Tv(l0 + threadIdx.x)[-1] = -0.0;
+        }
+    }
+    __syncthreads();
+    TailCell t[kMgTailCells];
+    const bool wave0 = threadIdx.x < kWave;
+    // the phases of a level of one wave's cells are ordered by the wave's
+    // in-order LDS accesses; __syncthreads joins it with the other waves
+    auto sync = [&](bool small) {
+        if (small)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        else
+            __syncthreads();
+    };
+    // down: nu sweeps from zero, the residual, and its sums over the children
+    int l = l0;
+    for (; l < last; ++l) {
+        const int n = T->lev[l].ncell;
+        const bool small = n <= kWave;
+        if (small && !wave0)
+            break; // wave 0 goes on alone
+        double *x = X(l), *u = Tv(l), *bv = Bv(l);
         const double* bg = T->B[l0];
-        double* b = Bv(l0);
-        CF_BLOCK_STRIDE(id, T->lev[l0].ncell) { b[id] = bg[id]; }
-        __syncthreads();
-    }
-    // down: pre-smoothing and restriction; the coarsest level in wave 0
-    for (int l = l0; l <= last; ++l) {
-        const MgLev L = T->lev[l];
-        const MgLev& C = L; // unused parent level of the non-prolong sweeps
-        const double* b = Bv(l);
-        if (l == last) {
-            if (threadIdx.x < kWave)
-                mg_coarsest_wave(L, b, res(l), coarse);
-            __syncthreads();
-            break;
-        }
-        double* x = X(l);
-        double* t = Tv(l);
-        const int pre = nu;
-        if (pre == 1) {
-            CF_BLOCK_STRIDE(id, L.ncell) { mg_first_cell(L, id, b, x); }
-        } else {
-            CF_BLOCK_STRIDE(id, L.ncell) { mg_smooth_cell<MG_FIRST>(L, id, nullptr, b, C, nullptr, x); }
-        }
-        __syncthreads();
-        for (int it = 2; it < pre; ++it) {
-            CF_BLOCK_STRIDE(id, L.ncell) { mg_smooth_cell<MG_PLAIN>(L, id, x, b, C, nullptr, t); }
-            __syncthreads();
-            double* tmp = x;
-            x = t;
-            t = tmp;
-        }
-        const MgLev Cn = T->lev[l + 1];
-        double* bn = Bv(l + 1);
-        CF_BLOCK_STRIDE(id, Cn.ncell) { mg_resrestrict_cell(L, Cn, id, x, b, bn); }
-        __syncthreads();
-    }
-    // up: prolongation fused into the first post-sweep
-    for (int l = last - 1; l >= l0; --l) {
-        const MgLev L = T->lev[l];
-        const MgLev Cn = T->lev[l + 1];
-        const double* b = Bv(l);
-        // the pre-smoothing result: X after an even number of swaps
-        const bool odd = (nu >= 2 ? nu - 2 : 0) & 1;
-        double* x = odd ? Tv(l) : X(l);
-        double* t = odd ? X(l) : Tv(l);
-        const double* xc = res(l + 1);
-        CF_BLOCK_STRIDE(id, L.ncell) { mg_smooth_cell<MG_PROLONG>(L, id, x, b, Cn, xc, t); }
-        __syncthreads();
-        double* tmp = x;
-        x = t;
-        t = tmp;
-        for (int it = 1; it < nu; ++it) {
-            CF_BLOCK_STRIDE(id, L.ncell) { mg_smooth_cell<MG_PLAIN>(L, id, x, b, L, nullptr, t); }
-            __syncthreads();
-            tmp = x;
-            x = t;
-            t = tmp;
+        const int fn0 = l > l0 ? T->lev[l - 1].n[0] : 0;
+        const int fn01 = l > l0 ? fn0 * T->lev[l - 1].n[1] : 0;
+        tail_each(n, t, [&](TailCell& c, int id) {
+            if (l == l0) {
+                c.b = bg[id];
+            }
+            const MgTailInfo f = info(l, id);
+            if (l > l0)
+                c.b = tail_children(f, mg_tail_residual(X(l - 1), Tv(l - 1), nu), fn0, fn01);
+            tail_cell(ops + (l - l0), f, c);
+            c.x = c.w * c.b;
+            bv[id] = c.b;
+            x[id] = c.x;
+        });
+        sync(small);
+        for (int it = 1; it <= nu; ++it) {
+            // sweeps 2 .. nu, then the residual, each into the other vector
+            const bool sweep = it < nu;
+            tail_each(n, t, [&](TailCell& c, int id) {
+                const double r = c.b - tail_apply(c, dim, x);
+                if (sweep) {
+                    c.x = fma(c.w, r, c.x);
+                    u[id] = c.x;
+                } else {
+                    u[id] = r;
+                }
+            });
+            sync(small);
+            double* v = x;
+            x = u;
+            u = v;
         }
     }
-    {
-        const double* x = res(l0);
-        double* xg = T->res[l0];
-        CF_BLOCK_STRIDE(id, T->lev[l0].ncell) { xg[id] = x[id]; }
+    if (l == last && wave0) { // the coarsest level
+        const MgLev& L = T->lev[last];
+        double* b = Bv(last);
+        if ((int)threadIdx.x < L.ncell) {
+            double sum;
+            if (last > l0) {
+                const MgLev& F = T->lev[last - 1];
+                sum = tail_children(info(last, threadIdx.x),
+                                    mg_tail_residual(X(last - 1), Tv(last - 1), nu), F.n[0],
+                                    F.n[0] * F.n[1]);
+            } else {
+                sum = T->B[last][threadIdx.x];
+            }
+            b[threadIdx.x] = sum;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        mg_coarsest_wave(L, b, X(last), coarse);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (l0 == last) {
+        if ((int)threadIdx.x < T->lev[last].ncell)
+            T->res[last][threadIdx.x] = X(last)[threadIdx.x];
+        return;
+    }
+    // up: nu sweeps from x + alpha times the parent's result.  The levels of
+    // wave 0 first, then all waves together.
+    bool joined = T->lev[last - 1].ncell > kWave;
+    if (joined)
+        __syncthreads(); // the coarsest level's result
+    for (l = last - 1; l >= l0; --l) {
+        const int n = T->lev[l].ncell;
+        const bool small = n <= kWave;
+        if (!small && !joined) {
+            joined = true;
+            __syncthreads();
+        }
+        if (small && !wave0)
+            continue;
+        // the down leg left x in the vector that its residual is not in; the
+        // prolongated x replaces the residual
+        double* u = mg_tail_residual(X(l), Tv(l), nu);
+        double* x = u == X(l) ? Tv(l) : X(l);
+        const double* xc = X(l + 1); // every level's result
+        const double* bv = Bv(l);
+        double* out = T->res[l0];
+        tail_each(n, t, [&](TailCell& c, int id) {
+            const MgTailInfo f = info(l, id);
+            tail_cell(ops + (l - l0), f, c);
+            c.b = bv[id];
+            c.x = fma(alpha, xc[f.w & 0xffff], x[id]);
+            u[id] = c.x;
+        });
+        sync(small);
+        for (int it = 0; it < nu; ++it) {
+            double* v = x;
+            x = u; // the values, and where the sweep writes
+            u = v;
+            tail_each(n, t, [&](TailCell& c, int id) {
+                c.x = fma(c.w, c.b - tail_apply(c, dim, x), c.x);
+                if (l == l0 && it == nu - 1)
+                    out[id] = c.x;
+                else
+                    u[id] = c.x;
+            });
+            if (it < nu - 1 || l > l0)
+                sync(small);
+        }
     }
 }
 

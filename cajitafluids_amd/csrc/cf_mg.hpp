@@ -27,10 +27,13 @@ namespace cfmi
 {
 
 constexpr int kMgMaxLevels = 24;
-// The coarsest levels whose vectors (3 per level) fit this much LDS run
-// inside one workgroup (k_mg_tail).
-constexpr int kMgTailLdsBytes = 64 * 1024;
+// The coarsest levels whose vectors (3 per level), tables and infos fit this
+// much LDS, and whose largest leaves a thread at most kMgTailCells cells, run
+// inside one workgroup (k_mg_tail).  Against 64 KB, where 16^3 cells ran as
+// legs of their own: 256^3 V-cycle 15 us shorter.
+constexpr int kMgTailLdsBytes = 150 * 1024;
 constexpr int kMgTailThreads = 1024;
+constexpr int kMgTailCells = 4;
 
 // omega * (1 / diag) on level 0, by the cell's SOLID wall count.
 struct MgTab
@@ -52,19 +55,6 @@ struct MgLev
     double s;         // dt / (rho dx^2)
     double omega;
     double alpha;     // coarse-correction scale: x = fma(alpha, x_parent, x)
-};
-
-// The levels that k_mg_tail runs (l0 .. last): their LDS offsets (X, T, B
-// of level l from element off[l]), and the global arrays it reads (B[l0])
-// and writes (res[l0]).  Each level starts a cycle in X and ends it in X or
-// T by the parity of its sweep count.
-struct MgTail
-{
-    int l0, last, nu, coarse;
-    MgLev lev[kMgMaxLevels];
-    int off[kMgMaxLevels];
-    double* B[kMgMaxLevels];
-    double* res[kMgMaxLevels];
 };
 
 // Linear index of the parent of cell (i, j, k) in the next level's array:
@@ -90,6 +80,38 @@ struct MgOp
     MgOpTab<double> d;
     MgOpTab<float> f; // the FP64 entries rounded
 };
+
+// A cell of those levels: x, y, z hold the elements of its -/+ neighbours
+// along each axis in bits 0-12 and 13-25, counted from 1 (0: none, across a
+// wall); x its class (MgOpTab) in bits 26-31; y in bits 26-28 whether its box
+// has a second child along each axis; w its parent's element, and in bits
+// 16-31 its first child's.
+using MgTailInfo = int4;
+
+// The levels that k_mg_tail runs (l0 .. last): their LDS offsets (level l's
+// vectors from element off[l], the operator tables from off[last + 1], the
+// cells' infos after them), and the global arrays it reads (B[l0]) and writes
+// (res[l0]).
+struct MgTail
+{
+    int l0, last, nu, coarse;
+    MgLev lev[kMgMaxLevels];
+    int off[kMgMaxLevels + 1];
+    double* B[kMgMaxLevels];
+    double* res[kMgMaxLevels];
+    const MgOp* op;         // of every level
+    const MgTailInfo* info; // level l's cells from info_at[l]
+    int info_at[kMgMaxLevels + 1];
+};
+
+// Which of a level's two vectors k_mg_tail's downward leg leaves the residual
+// in: x = w b in X, then nu - 1 sweeps and the residual, alternating.  The
+// upward leg's nu sweeps from there end in X.
+template <class P>
+__host__ __device__ inline P mg_tail_residual(P X, P T, int nu)
+{
+    return nu & 1 ? T : X;
+}
 
 // One level's legs in a launch each (cf_mg_fused.hip): its cells and its
 // parents' storage, and the tiling.
@@ -247,6 +269,8 @@ class Multigrid
     std::vector<MgFused> _fz[2];
     bool fused(int l) const { return _fz[0][l].work > 0; }
     MgOp op_table(int l) const;
+    void tail_infos(int l, std::vector<MgTailInfo>& out) const;
+    size_t tail_lds(int l0) const;
     std::unique_ptr<Buffers> _buf;
 };
 

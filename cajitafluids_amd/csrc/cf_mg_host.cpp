@@ -38,11 +38,14 @@ struct Multigrid::Buffers
     std::vector<std::unique_ptr<DevArray<double>>> vec;
     std::vector<double*> X, T, B, res;
     MgTail* tail = nullptr; // device copy
+    MgTailInfo* info = nullptr; // its cells, device
     MgOp* op = nullptr;     // operator tables of the fused levels, device
     ~Buffers()
     {
         if (tail)
             (void)hipFree(tail);
+        if (info)
+            (void)hipFree(info);
         if (op)
             (void)hipFree(op);
     }
@@ -144,10 +147,8 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
     // the tail: the coarsest levels whose X, T, B fit the LDS budget
     _tail0 = last;
     {
-        int64_t cells = 0;
         for (int l = last; l >= 1; --l) {
-            cells += _lev[l].ncell;
-            if (3 * cells * (int64_t)sizeof(double) > kMgTailLdsBytes)
+            if (_lev[l].ncell > kMgTailCells * kMgTailThreads || tail_lds(l) > kMgTailLdsBytes)
                 break;
             _tail0 = l;
         }
@@ -226,12 +227,20 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
     // a fused level's upward leg ends in T
     for (int l = 0; l < nl; ++l)
         B.res[l] = fused(l) || (mg_level_swaps(l == last, _nu, _coarse) & 1) ? B.T[l] : B.X[l];
+    std::vector<MgOp> op(nl);
     if (last >= 1) {
+        for (int l = 0; l < last; ++l)
+            op[l] = op_table(l);
+        void* p = nullptr;
+        CF_HIP(hipMalloc(&p, nl * sizeof(MgOp)));
+        B.op = (MgOp*)p;
+        CF_HIP(hipMemcpyAsync(B.op, op.data(), nl * sizeof(MgOp), hipMemcpyHostToDevice, s));
         MgTail h{};
         h.l0 = _tail0;
         h.last = last;
         h.nu = _nu;
         h.coarse = _coarse;
+        h.op = B.op;
         int off = 0;
         for (int l = 0; l < nl; ++l) {
             h.lev[l] = _lev[l];
@@ -239,28 +248,89 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
             h.res[l] = B.res[l];
             h.off[l] = off;
             if (l >= _tail0)
-                off += 3 * _lev[l].ncell;
+                off += (3 * _lev[l].ncell + 3) / 2 * 2; // X, T with a slot each, B; even
         }
-        _tail_lds = (size_t)off * sizeof(double);
-        void* p = nullptr;
+        h.off[nl] = off;
+        _tail_lds = tail_lds(_tail0);
+        std::vector<MgTailInfo> info;
+        for (int l = 0; l < nl; ++l) {
+            h.info_at[l] = (int)info.size();
+            if (l >= _tail0)
+                tail_infos(l, info);
+        }
+        h.info_at[nl] = (int)info.size();
+        CF_HIP(hipMalloc(&p, info.size() * sizeof(MgTailInfo)));
+        B.info = (MgTailInfo*)p;
+        CF_HIP(hipMemcpyAsync(B.info, info.data(), info.size() * sizeof(MgTailInfo),
+                              hipMemcpyHostToDevice, s));
+        CF_HIP(hipStreamSynchronize(s)); // info is this block's
+        h.info = B.info;
         CF_HIP(hipMalloc(&p, sizeof(MgTail)));
         B.tail = (MgTail*)p;
         CF_HIP(hipMemcpyAsync(B.tail, &h, sizeof(MgTail), hipMemcpyHostToDevice, s));
-    }
-    std::vector<MgOp> op(nl);
-    for (int l = 0; l < nl; ++l)
-        if (fused(l))
-            op[l] = op_table(l);
-    {
-        void* p = nullptr;
-        CF_HIP(hipMalloc(&p, nl * sizeof(MgOp)));
-        B.op = (MgOp*)p;
-        CF_HIP(hipMemcpyAsync(B.op, op.data(), nl * sizeof(MgOp), hipMemcpyHostToDevice, s));
     }
     CF_HIP(hipStreamSynchronize(s));
 }
 
 Multigrid::~Multigrid() = default;
+
+// LDS bytes of a tail from level l0 on: vectors (16-byte aligned), operator
+// tables, and the infos of the levels below l0.
+size_t Multigrid::tail_lds(int l0) const
+{
+    const int last = (int)_lev.size() - 1;
+    size_t b = (size_t)(last - l0) * sizeof(MgOpTab<double>);
+    for (int l = l0; l <= last; ++l)
+        b += (size_t)((3 * _lev[l].ncell + 3) / 2 * 2) * sizeof(double) +
+             (l > l0 ? (size_t)_lev[l].ncell * sizeof(MgTailInfo) : 0);
+    return b;
+}
+
+// Level l's cells for k_mg_tail.
+void Multigrid::tail_infos(int l, std::vector<MgTailInfo>& out) const
+{
+    const MgLev& L = _lev[l];
+    const bool leaf = l + 1 == (int)_lev.size(); // the coarsest level
+    for (int id = 0; id < L.ncell; ++id) {
+        const int c[3] = {id % L.n[0], id / L.n[0] % L.n[1], id / L.n[0] / L.n[1]};
+        const int stride[3] = {1, L.n[0], L.n[0] * L.n[1]};
+        unsigned nb[3], cls = 0, has = 0, parent = 0, child = 0;
+        int ps = 1, fs = 1;
+        for (int d = 0; d < 3; ++d) {
+            int e[2] = {0, 0};
+            for (int side = 0; side < 2 && d < L.dim; ++side) {
+                int m = c[d] + (side ? 1 : -1);
+                if (m < 0 || m >= L.n[d]) {
+                    if (!L.periodic[d])
+                        continue;
+                    m = m < 0 ? L.n[d] - 1 : 0;
+                }
+                e[side] = id + (m - c[d]) * stride[d] + 1;
+            }
+            nb[d] = (unsigned)e[0] | (unsigned)e[1] << 13;
+            if (d < L.dim)
+                cls |= (unsigned)((c[d] == 0 ? 1 : 0) + (c[d] == L.n[d] - 1 ? 2 : 0)) << (2 * d);
+            // the parent in the next level, the children in the last one
+            if (!leaf) {
+                parent += (unsigned)((L.coarsen[d] ? c[d] >> 1 : c[d]) * ps);
+                ps *= _lev[l + 1].n[d];
+            }
+            if (l > 0 && l > _tail0) {
+                const MgLev& F = _lev[l - 1];
+                const int lo = F.coarsen[d] ? 2 * c[d] : c[d];
+                has |= F.coarsen[d] && lo + 1 < F.n[d] ? 1u << d : 0u;
+                child += (unsigned)(lo * fs);
+                fs *= F.n[d];
+            }
+        }
+        MgTailInfo t;
+        t.x = (int)(nb[0] | cls << 26);
+        t.y = (int)(nb[1] | has << 26);
+        t.z = (int)nb[2];
+        t.w = (int)(parent | child << 16);
+        out.push_back(t);
+    }
+}
 
 // The operator of level l by class (MgOpTab): the entries its sweep kernels
 // read from their tables (padded levels) or compute (compact ones).

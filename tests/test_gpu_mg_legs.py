@@ -1,7 +1,8 @@
 """The multigrid legs that run a level's sweeps in one launch, against the
 oracle's V-cycle sweep by sweep: grids at the edges of the blocks (64 columns,
 24 and 32 rows, two-plane chunks), smaller than the overlap, odd and periodic,
-with two and three sweeps, in FP64 and with the FP32 finest levels.  Solves
+with two and three sweeps (and four, which run one by one but in the small
+levels), in FP64 and with the FP32 finest levels.  Solves
 stopped after two iterations, so that x holds two V-cycles and no limit."""
 import numpy as np
 import pytest
@@ -21,7 +22,7 @@ GRIDS = [
 
 
 @pytest.mark.parametrize("precision", [K.FP64, K.FP32_REFINED])
-@pytest.mark.parametrize("nu", [2, 3])
+@pytest.mark.parametrize("nu", [2, 3, 4])
 @pytest.mark.parametrize("n,periodic", GRIDS)
 def test_mg_legs(oracle_mod, n, periodic, nu, precision):
     from cajitafluids_amd import _lib
