@@ -128,15 +128,16 @@ int reduction_blocks_max(const Geo& g);
 // iterations of this launch (x, r and the direction p are read at the start
 // and written back at the end, so launches chain).  The same x, r, direction
 // and state bits as the dir_spmv / update pair.  pcg_coop_fits: the grid
-// qualifies (2-D, at most 2048 cells along x and 256 strips of 2048 cells);
-// xch: coop_xch_bytes(g) bytes of device memory.  A launch that waited too
+// qualifies (2-D, at most 256 strips of whole rows and 4096 cells);
+// xch: coop_xch_bytes(g) bytes of device memory, zero at first; seq: the last
+// exchange number used there (0 at first), advanced by the call.  A launch that waited too
 // long for another workgroup sets PcgState::stalled.  Returns false when the
 // runtime refuses the cooperative launch (the workgroups cannot all be
 // resident, or the device has no cooperative launch); nothing ran then.
 bool pcg_coop_fits(const Geo& g);
 size_t coop_xch_bytes(const Geo& g);
 bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgState* st,
-                           void* xch, int max_its, hipStream_t s);
+                           void* xch, unsigned& seq, int max_its, hipStream_t s);
 
 // FP32-inner / FP64-outer defect correction.  The host runs the outer loop
 // from the device-computed norms (one read-back per pass).

@@ -1,0 +1,620 @@
+// cf_pcg_coop.hip -- a whole FP64 PCG solve of a 2-D grid in one cooperative
+// launch.
+//
+// A 2-D streaming iteration at 128^2-512^2 is two launches whose time goes
+// to start-up, one sweep per lane group and the grid reduction's arrival
+// chain (about 7.5 us each at 128^2), not to bandwidth.  Here one
+// cooperative launch of G workgroups runs all iterations:
+//   - workgroup g owns the rows [g R, g R + R) as a strip; lane t of it owns
+//     strip cells t + NT m (m < CPT, x fastest); r, x and q = A p of those
+//     cells stay in registers;
+//   - the direction lives in the strip's LDS window: its rows, one halo row
+//     above and below, and a one-cell ring in x.  Ring cells of periodic
+//     axes are copies of the wrapped cells; the others hold a zero whose
+//     sign is that of the coupling s, so that fma(s, ring, y) adds
+//     s * ring = +0, the term fma(0, 0, y) the streaming kernels add across a
+//     non-periodic boundary (the same bits for every y, -0 included);
+//   - a halo row's direction is computed by the strip itself, by the same
+//     expression, from its last one and the neighbour strip's boundary r,
+//     which that strip publishes with the reduction below;
+//   - each of an iteration's two reductions: a workgroup reduction, then the
+//     workgroup's double-double partial published and every workgroup's
+//     partials read and summed in one fixed order, so that every workgroup
+//     holds the same alpha, beta and stop decision.
+//
+// What bounds it is the two exchanges' latency: a value travels as 64-bit
+// words of 32 bits of it and the exchange's sequence number, stored and
+// loaded at agent scope (past the L2s, which do not see each other's
+// writes), and its readers poll the words themselves.  No store's completion
+// is waited for, no separate flag is read, no fence is issued.  Measured per
+// exchange (16 workgroups): 2.7 us with a flag per workgroup (store, its
+// acknowledgement, flag, flag's poll, then the value's read), 2.1 us with the
+// words, 1.9 us with the wave sums by lane moves instead of LDS permutes,
+// 1.65 us with the workgroups on one XCD (every eighth block of the launch,
+// while that many fit the GPU; the others return at once, and nothing but
+// the latency depends on where the blocks really run).
+//
+// Every value is the streaming kernels' expression on the same operands, so
+// x, r, the direction and the state come out with the same bits.  A poll
+// that exceeds its bound sets PcgState::stalled and ends the launch (the
+// host reports CF_EDEVICE).
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "cf_pcg_state.hpp"
+#include "cf_solver.hpp"
+#include "cf_stream.hpp"
+
+namespace cfmi
+{
+
+namespace
+{
+
+constexpr int kCoopMaxGroups = 256;
+constexpr unsigned kCoopSpin = 1u << 22; // polls (about 1 us each) before a wait counts as stalled
+
+// Strip layout: R rows per strip, G strips; window row pitch e0 = n0 + 2
+// (window index of strip-relative cell (i, jj), halo rows jj = -1 and
+// jj = R: (i+1) + e0 (jj+1)).
+struct CoopGrid
+{
+    int G, R, e0, nwin;
+    int c00; // padded index of owned cell (0, 0)
+    int px;
+    int nt, cpt; // lanes per workgroup and cells per lane
+    int every;   // the strips are the launch's blocks 0, every, 2 every, ...
+};
+
+// The strips' shape: 4 cells a lane of 256 lanes while that makes at most 64
+// strips (one partial a lane of the gather), 4 of 512 up to 128 strips (two a
+// lane), else 8 of 512.  Fewer, larger strips shorten the exchanges and
+// lengthen the strip's own chain.  us per iteration at (256, 4), (512, 4),
+// (512, 8): 32^2 2.9 (one strip), 3.8, 5.0; 128^2 5.7, 5.8, 6.7; 256^2 6.8,
+// 7.7, 8.4; 391 x 263 9.7, 7.7, 9.0; 512^2 13.4, 9.1, 9.4; 700 x 500 -, 14.9,
+// 10.5; 1024^2 -, -, 16.9 (the streaming kernels 32.2).  1024 lanes, and 2
+// cells a lane, were slower or within 2% everywhere.
+CoopGrid coop_grid(const Geo& g)
+{
+    constexpr int shape[3][3] = {{256, 4, 64}, {512, 4, 128}, {512, 8, kCoopMaxGroups}};
+    CoopGrid cg;
+    for (const auto& sh : shape) {
+        cg.nt = sh[0];
+        cg.cpt = sh[1];
+        cg.R = cg.nt * cg.cpt / g.n[0];
+        if (cg.R > g.n[1])
+            cg.R = g.n[1];
+        cg.G = cg.R > 0 ? (g.n[1] + cg.R - 1) / cg.R : INT_MAX;
+        if (cg.G <= sh[2])
+            break;
+    }
+    cg.every = cg.G > 1 && cg.G <= 32 ? 8 : 1;
+    cg.e0 = g.n[0] + 2;
+    cg.nwin = cg.e0 * (cg.R + 2);
+    cg.c00 = (int)g.idx(g.h, g.h, g.own_lo(2));
+    cg.px = (int)g.px;
+    return cg;
+}
+
+// Bytes of LDS: the window, the coefficient tables, the halo rows' r and D^-1.
+size_t coop_lds(const Geo& g, const CoopGrid& cg)
+{
+    return ((size_t)cg.nwin + 14 + 4 * (size_t)g.n[0]) * sizeof(double);
+}
+
+using Word = unsigned long long;
+
+// The exchange buffer: per strip 16 words of partials (p.q in words 0-3,
+// r.r and r.z in 8-15), and per strip the two boundary rows' r, two words a
+// cell (top row, then bottom row).
+struct CoopXch
+{
+    Word* part; // [G][16]
+    Word* halo; // [G][2][n0][2]
+    unsigned seq0; // the launch's exchanges are numbered from seq0 + 1
+};
+
+__device__ __forceinline__ void put_word(Word* p, unsigned seq, unsigned v)
+{
+    __hip_atomic_store(p, (Word)seq << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ Word get_word(const Word* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double value_of(Word lo, Word hi)
+{
+    return __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffu)));
+}
+
+// A lane's value from lane ^ 1, ^ 2, and (where lanes of a quad, then of
+// eight, hold the same) from the other quad of eight and the other eight of
+// sixteen; from lane ^ 16 and ^ 32.
+template <int CTRL>
+__device__ __forceinline__ double move_row(double v)
+{
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+template <int W>
+__device__ __forceinline__ double move_half(double v)
+{
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    const bool up = (threadIdx.x & W) != 0;
+    if constexpr (W == 16) {
+        const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
+    } else {
+        const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
+    }
+}
+
+// Sums NV double-double values over groups of `width` lanes (a power of two),
+// the result in each of them.
+template <int NV>
+__device__ __forceinline__ void wave_sum(double (&hi)[NV], double (&lo)[NV], int width)
+{
+#define CF_STEP(W, MOVE)                                  \
+    if (width > W) {                                      \
+        _Pragma("unroll") for (int v = 0; v < NV; ++v)    \
+        {                                                 \
+            const double oh = MOVE(hi[v]), ol = MOVE(lo[v]); \
+            dd_add(hi[v], lo[v], oh, ol);                 \
+        }                                                 \
+    }
+    CF_STEP(1, move_row<0xB1>)  // quad_perm 1 0 3 2
+    CF_STEP(2, move_row<0x4E>)  // quad_perm 2 3 0 1
+    CF_STEP(4, move_row<0x141>) // row_half_mirror
+    CF_STEP(8, move_row<0x140>) // row_mirror
+    CF_STEP(16, move_half<16>)
+    CF_STEP(32, move_half<32>)
+#undef CF_STEP
+}
+
+// One reduction of the strip's lanes' NV sums over all strips: the workgroup
+// sum, its publication, and in wave 0 the rounded totals.  Wave 0 returns
+// with out set; the other waves return after the workgroup's barrier.
+// PPL: strips per lane of wave 0's gather.
+// shadow(): work that every wave does while the words travel.
+template <int NT, int NV, int PPL, class F>
+__device__ __forceinline__ void coop_reduce(double (&hi)[NV], double (&lo)[NV], int gid, int G,
+                                            Word* part, int off, unsigned seq,
+                                            double (*red)[2][NT / kWave], int* stall,
+                                            double (&out)[NV], F&& shadow)
+{
+    constexpr int NW = NT / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+        dd_norm(hi[v], lo[v]);
+    wave_sum<NV>(hi, lo, kWave);
+    if (lane == 0) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            red[v][0][wv] = hi[v];
+            red[v][1][wv] = lo[v];
+        }
+    }
+    __syncthreads();
+    if (wv != 0) {
+        shadow();
+        return;
+    }
+    double h[NV], l[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        h[v] = red[v][0][lane & (NW - 1)];
+        l[v] = red[v][1][lane & (NW - 1)];
+    }
+    wave_sum<NV>(h, l, NW);
+    if (G > 1) {
+        if (lane < 4 * NV) { // word lane & 3 of value lane >> 2
+            const double a = NV > 1 && lane >= 4 ? h[NV - 1] : h[0];
+            const double b = NV > 1 && lane >= 4 ? l[NV - 1] : l[0];
+            const double v = lane & 2 ? b : a;
+            put_word(part + (size_t)gid * 16 + off + lane, seq,
+                     (unsigned)(lane & 1 ? __double2hiint(v) : __double2loint(v)));
+        }
+        shadow();
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+            h[v] = l[v] = 0.0;
+        Word w[PPL][4 * NV];
+        unsigned polls = 0;
+        for (;;) {
+            bool all = true;
+#pragma unroll
+            for (int u = 0; u < PPL; ++u) {
+                const int q = lane + kWave * u;
+                const Word* pq = part + (size_t)(q < G ? q : 0) * 16 + off;
+#pragma unroll
+                for (int k = 0; k < 4 * NV; ++k)
+                    w[u][k] = get_word(pq + k);
+            }
+#pragma unroll
+            for (int u = 0; u < PPL; ++u)
+#pragma unroll
+                for (int k = 0; k < 4 * NV; ++k)
+                    all = all && (unsigned)(w[u][k] >> 32) == seq;
+            if (__all(all))
+                break;
+            if (++polls >= kCoopSpin) {
+                if (lane == 0)
+                    *stall = 1;
+                break;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < PPL; ++u)
+            if (lane + kWave * u < G) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v)
+                    dd_add(h[v], l[v], value_of(w[u][4 * v], w[u][4 * v + 1]),
+                           value_of(w[u][4 * v + 2], w[u][4 * v + 3]));
+            }
+        wave_sum<NV>(h, l, G < kWave ? 1 << (32 - __builtin_clz(G - 1)) : kWave);
+    } else {
+        shadow();
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+        out[v] = h[v] + l[v];
+}
+
+// Bits of a lane's cell slots: owned (a slot past the strip's last cell is
+// not, and carries the first cell's window index; its stores and sums are
+// masked), and in the strip's top / bottom row.
+struct CoopSlots
+{
+    unsigned own, top, bottom;
+};
+
+template <int NT, int CPT, int PPL>
+__global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, double* __restrict__ x,
+                                                       double* __restrict__ r,
+                                                       double* __restrict__ pg, PcgState* st,
+                                                       CoopXch xc, int max_its)
+{
+    if (blockIdx.x % cg.every)
+        return;
+    extern __shared__ double lds[];
+    double* pw = lds;             // the direction window
+    double* tab = lds + cg.nwin;  // diag[0..6], then dinv[0..6]
+    double* hr = tab + 14;        // halo rows' r [2][n0]
+    double* hd = hr + 2 * g.n[0]; // and their D^-1
+    __shared__ double red[2][2][NT / kWave];
+    __shared__ double sh_ab[2]; // alpha, beta
+    __shared__ int sh_stop, sh_stall;
+    // The state is read once, here; thread 0 of every workgroup keeps the same
+    // copy in registers, and workgroup 0 stores it back at the end.  A read
+    // of *st after a write in this kernel could be served by the scalar
+    // cache, which vector stores do not update.
+    PcgState fs = *st;
+    const int t = threadIdx.x;
+    const int gid = blockIdx.x / cg.every, G = cg.G;
+    const int n0 = g.n[0], n1 = g.n[1], e0 = cg.e0;
+    const int j0 = gid * cg.R;
+    const int nrows = (j0 + cg.R < n1 ? cg.R : n1 - j0);
+    const double s = offdiag<double>(g);
+    const double ring0 = copysign(0.0, s);
+    if (t == 0)
+        sh_stall = 0;
+    for (int e = t; e < cg.nwin; e += NT)
+        pw[e] = ring0;
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        if (t == q) {
+            tab[q] = g.diag[q];
+            tab[7 + q] = g.dinv[q];
+        }
+    __syncthreads();
+    if (fs.done)
+        return;
+    bool first = fs.iter == 0;
+    double beta = fs.beta;
+
+    // halo rows: window rows 0 (global row j0 - 1) and nrows + 1 (row j0 +
+    // nrows), when they exist; gtop / gbot the strips that own them
+    const bool py = g.periodic[1];
+    const bool has_top = j0 > 0 || py, has_bot = j0 + nrows < n1 || py;
+    const int jtop = j0 > 0 ? j0 - 1 : n1 - 1, jbot = j0 + nrows < n1 ? j0 + nrows : 0;
+    const int gtop = gid > 0 ? gid - 1 : G - 1, gbot = gid + 1 < G ? gid + 1 : 0;
+    // SOLID wall count of a cell of global row j (in 2-D, z adds its own
+    // count for k = 0 as the streaming kernels do)
+    auto cell_cnt = [&](int i, int j) -> int { return row_stencil(g, j, 0).cnt + lane_x(g, i).cnt; };
+    // window index of a halo cell
+    auto halo_at = [&](int side, int i) -> int { return (i + 1) + (side == 0 ? 0 : e0 * (nrows + 1)); };
+    // the two halo rows' r, and a resumed solve's direction, from the padded
+    // arrays (start of a launch)
+    for (int e = t; e < 2 * n0; e += NT) {
+        const int side = e >= n0 ? 1 : 0, i = e - side * n0;
+        if (side == 0 ? has_top : has_bot) {
+            const int64_t c = cg.c00 + i + (int64_t)cg.px * (side == 0 ? jtop : jbot);
+            hr[e] = r[c];
+            hd[e] = tab[7 + cell_cnt(i, side == 0 ? jtop : jbot)];
+            if (!first)
+                pw[halo_at(side, i)] = pg[c];
+        }
+    }
+
+    int wi[CPT]; // window indices
+    double rv[CPT], qv[CPT], xv[CPT], dg[CPT], dv[CPT];
+    CoopSlots sl{0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < CPT; ++m) {
+        const int L = t + NT * m;
+        const int i = L % n0, jj = L / n0;
+        wi[m] = 1 + e0; // strip cell (0, 0)
+        rv[m] = 0.0;
+        qv[m] = 0.0;
+        xv[m] = 0.0;
+        dg[m] = tab[0];
+        dv[m] = tab[7];
+        if (jj < nrows) {
+            const int cnt = cell_cnt(i, j0 + jj);
+            wi[m] = (i + 1) + e0 * (jj + 1);
+            dg[m] = tab[cnt];
+            dv[m] = tab[7 + cnt];
+            sl.own |= 1u << m;
+            sl.top |= jj == 0 ? 1u << m : 0u;
+            sl.bottom |= jj == nrows - 1 ? 1u << m : 0u;
+            const int64_t c = cg.c00 + i + (int64_t)cg.px * (j0 + jj);
+            rv[m] = r[c];
+            xv[m] = x[c];
+            if (!first)
+                pw[wi[m]] = pg[c];
+        }
+    }
+    // padded index of a slot's cell
+    auto padded = [&](int li) -> int64_t {
+        const int jj = li / e0 - 1, i = li - e0 * (jj + 1) - 1;
+        return cg.c00 + i + (int64_t)cg.px * (j0 + jj);
+    };
+    __syncthreads();
+    unsigned seq = xc.seq0;
+    for (int its = 1;; ++its) {
+        // direction: p = D^-1 r, or fma(beta, p, D^-1 r), for the strip's
+        // cells and its halo rows
+        double pn[CPT];
+#pragma unroll
+        for (int m = 0; m < CPT; ++m)
+            pn[m] = pw[wi[m]];
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double z = dv[m] * rv[m];
+            pn[m] = first ? z : fma(beta, pn[m], z);
+        }
+#pragma unroll
+        for (int m = 0; m < CPT; ++m)
+            if (sl.own >> m & 1)
+                pw[wi[m]] = pn[m];
+        for (int e = t; e < 2 * n0; e += NT) {
+            const int side = e >= n0 ? 1 : 0, i = e - side * n0;
+            if (side == 0 ? has_top : has_bot) {
+                const double z = hd[e] * hr[e];
+                double* pp = pw + halo_at(side, i);
+                *pp = first ? z : fma(beta, *pp, z);
+            }
+        }
+        __syncthreads();
+        if (g.periodic[0]) {
+            for (int jw = t; jw < nrows + 2; jw += NT) {
+                double* row = pw + e0 * jw;
+                row[0] = row[n0];
+                row[n0 + 1] = row[1];
+            }
+            __syncthreads();
+        }
+        // q = A p in the stencil order {0}, -x, +x, -y, +y; p.q
+        double h1[1] = {0.0}, l1[1] = {0.0};
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double* pp = pw + wi[m];
+            const bool own = sl.own >> m & 1;
+            const double pc = own ? pn[m] : 0.0;
+            double y = dg[m] * pn[m];
+            y = fma(s, pp[-1], y);
+            y = fma(s, pp[1], y);
+            y = fma(s, pp[-e0], y);
+            y = fma(s, pp[e0], y);
+            qv[m] = own ? y : 0.0;
+            dd_acc_prod(h1[0], l1[0], pc, qv[m]);
+        }
+        {
+            double pq[1];
+            coop_reduce<NT, 1, PPL>(h1, l1, gid, G, xc.part, 0, ++seq, red, &sh_stall, pq, [] {});
+            if (t == 0) {
+                fs.alpha = fs.rho / pq[0];
+                sh_ab[0] = fs.alpha;
+            }
+        }
+        __syncthreads();
+        if (sh_stall)
+            break;
+        const double alpha = sh_ab[0];
+        // x = fma(alpha, p, x); r = fma(-alpha, q, r); r.r and r.(D^-1 r).
+        // Past the strip's last cell q = r = 0, so rn = 0 and the sums are
+        // unchanged.
+        double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
+        ++seq;
+#pragma unroll
+        for (int m = 0; m < CPT; ++m)
+            rv[m] = fma(-alpha, qv[m], rv[m]);
+        // boundary rows' new r for the neighbour strips (the one strip of a
+        // periodic axis is its own)
+        if (sl.top | sl.bottom) {
+#pragma unroll
+            for (int m = 0; m < CPT; ++m) {
+                const unsigned side2 = (sl.top >> m & 1) | (sl.bottom >> m & 1) << 1;
+                if (!side2)
+                    continue;
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    if (!(side2 >> side & 1))
+                        continue;
+                    const int i = wi[m] - 1 - e0 * (side == 0 ? 1 : nrows);
+                    if (G > 1) {
+                        Word* hb = xc.halo + (((size_t)gid * 2 + side) * n0 + i) * 2;
+                        put_word(hb, seq, (unsigned)__double2loint(rv[m]));
+                        put_word(hb + 1, seq, (unsigned)__double2hiint(rv[m]));
+                    } else {
+                        hr[(side ^ 1) * n0 + i] = rv[m];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double z = dv[m] * rv[m];
+            dd_acc_prod(hi[0], lo[0], rv[m], rv[m]);
+            dd_acc_prod(hi[1], lo[1], rv[m], z);
+        }
+        {
+            double rr[2];
+            coop_reduce<NT, 2, PPL>(hi, lo, gid, G, xc.part, 8, seq, red, &sh_stall, rr, [&] {
+#pragma unroll
+                for (int m = 0; m < CPT; ++m)
+                    xv[m] = fma(alpha, pn[m], xv[m]);
+            });
+            if (t == 0) {
+                finish_update(&fs, rr[0], rr[1]);
+                sh_stop = fs.done || its >= max_its;
+                sh_ab[1] = fs.beta;
+            }
+        }
+        if (G > 1 && t >= kWave) {
+            // the other waves: the neighbours' boundary rows, a few cells a
+            // lane at a time so that their words are in flight together
+            constexpr int NB = 4;
+            constexpr int NH = NT - kWave;
+            for (int e1 = t - kWave; e1 < 2 * n0; e1 += NB * NH) {
+                Word w[NB][2];
+                unsigned polls = 0;
+                for (;;) {
+                    bool all = true;
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        const int e = e1 + b * NH;
+                        const int side = e >= n0 ? 1 : 0, i = e - side * n0;
+                        const bool want = e < 2 * n0 && (side == 0 ? has_top : has_bot);
+                        // the top halo row is the bottom row of the strip above
+                        const Word* hb =
+                            xc.halo + (want ? (((size_t)(side == 0 ? gtop : gbot) * 2 +
+                                                (side == 0 ? 1 : 0)) * n0 + i) * 2
+                                            : 0);
+                        w[b][0] = get_word(hb);
+                        w[b][1] = get_word(hb + 1);
+                        if (!want)
+                            w[b][0] = w[b][1] = (Word)seq << 32;
+                    }
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        all = all && (unsigned)(w[b][0] >> 32) == seq &&
+                              (unsigned)(w[b][1] >> 32) == seq;
+                    if (all)
+                        break;
+                    if (++polls >= kCoopSpin) {
+                        sh_stall = 1;
+                        break;
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    if (e1 + b * NH < 2 * n0)
+                        hr[e1 + b * NH] = value_of(w[b][0], w[b][1]);
+            }
+        }
+        __syncthreads();
+        if (sh_stall || sh_stop)
+            break;
+        beta = sh_ab[1];
+        first = false;
+    }
+    // x, r and the direction back to memory (a later launch resumes from
+    // them), and the state from workgroup 0
+    if (sh_stall)
+        fs.stalled = 1;
+    if (gid == 0 && t == 0)
+        *st = fs;
+#pragma unroll
+    for (int m = 0; m < CPT; ++m)
+        if (sl.own >> m & 1) {
+            const int64_t c = padded(wi[m]);
+            x[c] = xv[m];
+            r[c] = rv[m];
+            pg[c] = pw[wi[m]];
+        }
+}
+
+template <int NT, int CPT>
+const void* coop_kernel(int G)
+{
+    static_assert(kCoopMaxGroups <= 4 * kWave, "gather bucket");
+    return G <= kWave       ? (const void*)k_pcg_solve_coop<NT, CPT, 1>
+           : G <= 2 * kWave ? (const void*)k_pcg_solve_coop<NT, CPT, 2>
+                            : (const void*)k_pcg_solve_coop<NT, CPT, 4>;
+}
+
+} // namespace
+
+bool pcg_coop_fits(const Geo& g)
+{
+    if (g.dim != 2)
+        return false;
+    const CoopGrid cg = coop_grid(g);
+    if (cg.G > kCoopMaxGroups)
+        return false;
+    // window indices fit the slot word's 16 bits
+    return cg.nwin < (1 << 16) && coop_lds(g, cg) <= 128 * 1024;
+}
+
+size_t coop_xch_bytes(const Geo& g)
+{
+    const CoopGrid cg = coop_grid(g);
+    return (size_t)cg.G * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
+}
+
+bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgState* st,
+                           void* xch, unsigned& seq, int max_its, hipStream_t s)
+{
+    if (!pcg_coop_fits(g))
+        throw CfError(CF_EINVAL, "grid does not fit the cooperative PCG");
+    if (max_its < 1)
+        throw CfError(CF_EINVAL, "the cooperative PCG runs at least one iteration per launch");
+    const CoopGrid cg = coop_grid(g);
+    // a word is new when it carries its exchange's number: the numbers go on
+    // from launch to launch, and before they wrap the buffer is cleared
+    if (seq > 0xffffffffu - 2u * (unsigned)max_its - 2u) {
+        CF_HIP(hipMemsetAsync(xch, 0, coop_xch_bytes(g), s));
+        seq = 0;
+    }
+    CoopXch xc;
+    xc.part = (Word*)xch;
+    xc.halo = xc.part + (size_t)cg.G * 16;
+    xc.seq0 = seq;
+    Geo ga = g;
+    CoopGrid cga = cg;
+    double *xa = x, *ra = r, *pa = p;
+    PcgState* sta = st;
+    int ma = max_its;
+    void* args[] = {&ga, &cga, &xa, &ra, &pa, &sta, &xc, &ma};
+    const void* fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
+         : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
+                       : coop_kernel<512, 8>(cg.G);
+    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(cg.G * cg.every), dim3(cg.nt), args,
+                                                    (unsigned)coop_lds(g, cg), s);
+    if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
+        (void)hipGetLastError(); // refused before anything ran
+        return false;
+    }
+    CF_HIP(e);
+    seq += 2u * (unsigned)max_its;
+    return true;
+}
+
+} // namespace cfmi

@@ -359,7 +359,7 @@ int VelocityCorrector::runCoop(double* x)
     for (;; its = kCoopItsPerLaunch) {
         const int t0 = _timer.begin(_s);
         const bool ran = launch_pcg_solve_coop(pcgGeo(), x, _r.ptr, _p[0].ptr, _st, _xch.ptr,
-                                               its, _s);
+                                               _xch_seq, its, _s);
         _timer.end(t0, _s, TK_PCG_COOP, 0);
         if (!ran) {
             _timer.resolve(INT_MAX);

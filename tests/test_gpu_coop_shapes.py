@@ -1,0 +1,56 @@
+"""The cooperative 2-D solve over its strip shapes: one strip, the last row of
+a shape's range and the first of the next, one to four partials a lane of the
+gather, rows of more than 2048 cells, and strips on every eighth block of the
+launch or on all; x bit for bit the oracle's after an odd and an even number
+of iterations, and across two launches."""
+import numpy as np
+import pytest
+
+from cajitafluids_amd import configs as K
+from helpers import gpu_to_oracle
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    ((32, 32), (1, 1)), ((33, 31), (0, 0)), ((31, 34), (0, 1)), ((5, 3), (0, 0)),
+    ((128, 256), (0, 0)), ((128, 257), (0, 1)), ((256, 256), (1, 0)), ((256, 257), (0, 0)),
+    ((1024, 64), (0, 0)), ((1025, 40), (1, 1)), ((600, 600), (0, 0)), ((1200, 700), (0, 1)),
+    ((2300, 30), (0, 0)),
+]
+
+
+@pytest.mark.parametrize("n,periodic", SHAPES)
+@pytest.mark.parametrize("maxit", [1, 4, 259])
+def test_coop_shapes(oracle_mod, n, periodic, maxit):
+    from cajitafluids_amd import _lib
+    from cajitafluids_amd.solver import Solver
+    if maxit > 4 and n[0] * n[1] > 70000:
+        pytest.skip("two launches: on the smaller grids")
+    cfg = K.base_config(2, n[0])
+    cfg.update(num_cell=[n[0], n[1], 1], hi=[1.0, n[1] / n[0], 1.0], clamp_dt=0, dt=0.002,
+               periodic=[periodic[0], periodic[1], 0], cg_max_iter=maxit, cg_tol=1e-300)
+    print(f"coop shapes: {n} {periodic} maxit {maxit}", flush=True)
+    sol, orc = Solver(cfg), oracle_mod.Oracle(cfg)
+    sol.set_kernel_timing(True)
+    sol.init_random_faces(5)
+    gpu_to_oracle(sol, orc)
+    for o in (sol, orc):
+        o.build_rhs()
+        o.rhs_remove_mean()
+    for _ in range(2):  # the second solve's exchanges follow the first's
+        try:
+            sol.pressure_solve(K.FP64)
+            code = 0
+        except _lib.CfError as e:
+            code = e.code
+    rc, st_o = orc.pressure_solve(K.FP64)
+    assert code == rc
+    assert sol.last_stats["iterations"] == st_o["iterations"]
+    assert sol.kernel_time(_lib.TK_PCG_COOP)[1] >= 2
+    assert sol.kernel_time(_lib.TK_DIR_SPMV)[1] == 0
+    x_g = sol.owned_view(sol.get_pressure(0), 0)
+    x_o = orc.owned_view(orc.lhs(), 0)
+    assert np.any(x_o != 0.0)
+    assert np.array_equal(x_g, x_o)
+    sol.close()
+    orc.close()
