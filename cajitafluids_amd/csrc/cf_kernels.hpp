@@ -123,12 +123,12 @@ inline bool pcg_pairs_x(const Geo& g)
 // partials buffer).
 int reduction_blocks_max(const Geo& g);
 
-// 2-D grids: FP64 Jacobi-PCG iterations in one cooperative launch of one
-// workgroup per strip of rows, until the state's stop test or `max_its`
+// FP64 Jacobi-PCG iterations in one cooperative launch of one workgroup per
+// strip of rows (2-D) or pencil of x-rows (3-D), until the state's stop test or `max_its`
 // iterations of this launch (x, r and the direction p are read at the start
 // and written back at the end, so launches chain).  The same x, r, direction
 // and state bits as the dir_spmv / update pair.  pcg_coop_fits: the grid
-// qualifies (2-D, at most 256 strips of whole rows and 4096 cells);
+// qualifies (at most 256 strips or pencils of whole rows and 4096 cells);
 // xch: coop_xch_bytes(g) bytes of device memory, zero at first; seq: the last
 // exchange number used there (0 at first), advanced by the call.  A launch that waited too
 // long for another workgroup sets PcgState::stalled.  Returns false when the

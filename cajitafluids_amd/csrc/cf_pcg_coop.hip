@@ -1,5 +1,5 @@
-// cf_pcg_coop.hip -- a whole FP64 PCG solve of a 2-D grid in one cooperative
-// launch.
+// cf_pcg_coop.hip -- a whole FP64 PCG solve of a 2-D grid, or of a 3-D grid of
+// up to about 100^3 cells, in one cooperative launch.
 //
 // A 2-D streaming iteration at 128^2-512^2 is two launches whose time goes
 // to start-up, one sweep per lane group and the grid reduction's arrival
@@ -41,6 +41,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <cmath>
 
 #include "cf_pcg_state.hpp"
 #include "cf_solver.hpp"
@@ -560,12 +561,370 @@ const void* coop_kernel(int G)
                             : (const void*)k_pcg_solve_coop<NT, CPT, 4>;
 }
 
+// ---- 3-D grids ------------------------------------------------------------------------
+// The same solve with a workgroup per pencil of by x bz whole x-rows.  The
+// window holds the pencil's rows and one row around them; a boundary cell's
+// new r goes out as two words at the cell's own place (a neighbour pencil
+// polls that place), so no pencil needs to know which one owns its halo.  A
+// halo cell's r stays in its lane's registers from the poll to the next
+// direction.  The wave that gathers the partials has no halo cells.
+struct Coop3Grid
+{
+    int G, by, bz, gy; // pencils, their rows along y and z, pencils along y
+    int e0, e1, nwin;  // window pitches (x row, plane) and size
+    int c00, px;       // padded index of owned cell (0, 0, 0), pitches
+    int64_t pxy;
+    int nt, cpt, every;
+};
+constexpr int kCoopHalo = 8; // halo cells per lane at most
+
+// A bit mask the compiler re-reads: its bits' tests are not all kept as lane
+// masks across the loop (which spilled the scalar registers).
+__device__ __forceinline__ unsigned fresh(unsigned v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <int NT, int CPT, int PPL>
+__global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
+                                                        double* __restrict__ x,
+                                                        double* __restrict__ r,
+                                                        double* __restrict__ pg, PcgState* st,
+                                                        CoopXch xc, int max_its)
+{
+    if (blockIdx.x % cg.every)
+        return;
+    extern __shared__ double lds[];
+    double* pw = lds;            // the direction window
+    double* tab = lds + cg.nwin; // diag[0..6], then dinv[0..6]
+    double* xl = tab + 14;       // x of the lane's cells, CPT per lane
+    __shared__ double red[2][2][NT / kWave];
+    __shared__ double sh_ab[2]; // alpha, beta
+    __shared__ int sh_stop, sh_stall;
+    PcgState fs = *st; // read once, as in k_pcg_solve_coop
+    const int t = threadIdx.x;
+    const int gid = blockIdx.x / cg.every, G = cg.G;
+    const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2], e0 = cg.e0, e1 = cg.e1;
+    const int j0 = gid % cg.gy * cg.by, k0 = gid / cg.gy * cg.bz;
+    const int nby = min(cg.by, n1 - j0), nbz = min(cg.bz, n2 - k0);
+    const double s = offdiag<double>(g);
+    const double ring0 = copysign(0.0, s);
+    if (t == 0)
+        sh_stall = 0;
+    for (int e = t; e < cg.nwin; e += NT)
+        pw[e] = ring0;
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        if (t == q) {
+            tab[q] = g.diag[q];
+            tab[7 + q] = g.dinv[q];
+        }
+    __syncthreads();
+    if (fs.done)
+        return;
+    bool first = fs.iter == 0;
+    double beta = fs.beta;
+    auto cell_cnt = [&](int i, int j, int k) -> int {
+        return wall_count(g, 0, i) + wall_count(g, 1, j) + wall_count(g, 2, k);
+    };
+    auto padded = [&](int i, int j, int k) -> int64_t {
+        return cg.c00 + i + (int64_t)cg.px * j + cg.pxy * k;
+    };
+
+    // halo cells: the rows y-low, y-high (nbz each), z-low, z-high (nby each).
+    // hw: window index (bits 0-15), SOLID wall count (bits 16-18), kept only
+    // where the row exists; hs: the cell's number.
+    constexpr int NH = NT - kWave;
+    const int nrow = 2 * (nby + nbz);
+    int hw[kCoopHalo], hs[kCoopHalo];
+    double hr[kCoopHalo];
+    unsigned halo_bits = 0;
+#pragma unroll
+    for (int b = 0; b < kCoopHalo; ++b) {
+        hw[b] = hs[b] = 0;
+        hr[b] = 0.0;
+        const int h = t - kWave + NH * b;
+        const int row = h / n0, i = h - row * n0;
+        if (t < kWave || row >= nrow)
+            continue;
+        int jj, kk; // pencil-relative
+        if (row < 2 * nbz) {
+            jj = row < nbz ? -1 : nby;
+            kk = row < nbz ? row : row - nbz;
+        } else {
+            const int q = row - 2 * nbz;
+            jj = q < nby ? q : q - nby;
+            kk = q < nby ? -1 : nbz;
+        }
+        int j = j0 + jj, k = k0 + kk;
+        if (j < 0 || j >= n1) {
+            if (!g.periodic[1])
+                continue;
+            j = j < 0 ? n1 - 1 : 0;
+        }
+        if (k < 0 || k >= n2) {
+            if (!g.periodic[2])
+                continue;
+            k = k < 0 ? n2 - 1 : 0;
+        }
+        halo_bits |= 1u << b;
+        const int w = (i + 1) + e0 * (jj + 1) + e1 * (kk + 1);
+        hw[b] = w | cell_cnt(i, j, k) << 16;
+        hs[b] = i + n0 * (j + n1 * k);
+        const int64_t c = padded(i, j, k);
+        hr[b] = r[c];
+        if (!first)
+            pw[w] = pg[c];
+    }
+
+    // own cells: window index, and SOLID wall count (bits 16-18)
+    int wi[CPT], no[CPT]; // no: the cell's number
+    double rv[CPT], qv[CPT];
+    unsigned own_bits = 0, edge_bits = 0; // edge: some pencil's halo
+    const int ncell = n0 * nby * nbz;
+#pragma unroll
+    for (int m = 0; m < CPT; ++m) {
+        wi[m] = 1 + e0 + e1; // pencil cell (0, 0, 0)
+        no[m] = 0;
+        rv[m] = qv[m] = 0.0;
+        const int L = t + NT * m;
+        if (L < ncell) {
+            const int row = L / n0, i = L - row * n0;
+            const int kk = row / nby, jj = row - kk * nby;
+            no[m] = i + n0 * (j0 + jj + n1 * (k0 + kk));
+            wi[m] = ((i + 1) + e0 * (jj + 1) + e1 * (kk + 1)) |
+                    cell_cnt(i, j0 + jj, k0 + kk) << 16;
+            own_bits |= 1u << m;
+            edge_bits |= jj == 0 || jj == nby - 1 || kk == 0 || kk == nbz - 1 ? 1u << m : 0u;
+            const int64_t c = padded(i, j0 + jj, k0 + kk);
+            rv[m] = r[c];
+            xl[L] = x[c];
+            if (!first)
+                pw[wi[m] & 0xffff] = pg[c];
+        }
+    }
+    __syncthreads();
+    unsigned seq = xc.seq0;
+    for (int its = 1;; ++its) {
+        const unsigned own = fresh(own_bits), edge = fresh(edge_bits), have = fresh(halo_bits);
+        // direction: p = D^-1 r, or fma(beta, p, D^-1 r), own and halo cells
+        double pn[CPT];
+#pragma unroll
+        for (int m = 0; m < CPT; ++m)
+            pn[m] = pw[wi[m] & 0xffff];
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double z = tab[7 + (wi[m] >> 16)] * rv[m];
+            pn[m] = first ? z : fma(beta, pn[m], z);
+        }
+#pragma unroll
+        for (int m = 0; m < CPT; ++m)
+            if (own >> m & 1)
+                pw[wi[m] & 0xffff] = pn[m];
+#pragma unroll
+        for (int b = 0; b < kCoopHalo; ++b)
+            if (have >> b & 1) {
+                const double z = tab[7 + (hw[b] >> 16)] * hr[b];
+                double* pp = pw + (hw[b] & 0xffff);
+                *pp = first ? z : fma(beta, *pp, z);
+            }
+        __syncthreads();
+        if (g.periodic[0]) {
+            for (int q = t; q < nby * nbz; q += NT) {
+                double* row = pw + e0 * (q % nby + 1) + e1 * (q / nby + 1);
+                row[0] = row[n0];
+                row[n0 + 1] = row[1];
+            }
+            __syncthreads();
+        }
+        // q = A p in the stencil order {0}, -x, +x, -y, +y, -z, +z; p.q
+        double h1[1] = {0.0}, l1[1] = {0.0};
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double* pp = pw + (wi[m] & 0xffff);
+            const bool mine = own >> m & 1;
+            double y = tab[wi[m] >> 16] * pn[m];
+            y = fma(s, pp[-1], y);
+            y = fma(s, pp[1], y);
+            y = fma(s, pp[-e0], y);
+            y = fma(s, pp[e0], y);
+            y = fma(s, pp[-e1], y);
+            y = fma(s, pp[e1], y);
+            qv[m] = mine ? y : 0.0;
+            dd_acc_prod(h1[0], l1[0], mine ? pn[m] : 0.0, qv[m]);
+        }
+        {
+            double pq[1];
+            coop_reduce<NT, 1, PPL>(h1, l1, gid, G, xc.part, 0, ++seq, red, &sh_stall, pq, [] {});
+            if (t == 0) {
+                fs.alpha = fs.rho / pq[0];
+                sh_ab[0] = fs.alpha;
+            }
+        }
+        __syncthreads();
+        if (sh_stall)
+            break;
+        const double alpha = sh_ab[0];
+        // r = fma(-alpha, q, r), published where a neighbour needs it; r.r and
+        // r.(D^-1 r); x = fma(alpha, p, x)
+        double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
+        ++seq;
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            rv[m] = fma(-alpha, qv[m], rv[m]);
+            if (edge >> m & 1) {
+                Word* hb = xc.halo + 2 * (size_t)no[m];
+                put_word(hb, seq, (unsigned)__double2loint(rv[m]));
+                put_word(hb + 1, seq, (unsigned)__double2hiint(rv[m]));
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < CPT; ++m) {
+            const double z = tab[7 + (wi[m] >> 16)] * rv[m];
+            dd_acc_prod(hi[0], lo[0], rv[m], rv[m]);
+            dd_acc_prod(hi[1], lo[1], rv[m], z);
+        }
+        {
+            double rr[2];
+            coop_reduce<NT, 2, PPL>(hi, lo, gid, G, xc.part, 8, seq, red, &sh_stall, rr, [&] {
+#pragma unroll
+                for (int m = 0; m < CPT; ++m)
+                    xl[t + NT * m] = fma(alpha, pw[wi[m] & 0xffff], xl[t + NT * m]);
+            });
+            if (t == 0) {
+                finish_update(&fs, rr[0], rr[1]);
+                sh_stop = fs.done || its >= max_its;
+                sh_ab[1] = fs.beta;
+            }
+        }
+        // the halo cells' new r (none in the gathering wave), four a lane at a
+        // time
+#pragma unroll
+        for (int b0 = 0; b0 < kCoopHalo; b0 += 4) {
+            if (!(have >> b0 & 15))
+                continue;
+            Word w[4][2];
+            unsigned polls = 0;
+            for (;;) {
+                bool all = true;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const Word* hb = xc.halo + 2 * (size_t)hs[b0 + b];
+                    w[b][0] = get_word(hb);
+                    w[b][1] = get_word(hb + 1);
+                }
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    all = all && (!(have >> (b0 + b) & 1) ||
+                                  ((unsigned)(w[b][0] >> 32) == seq &&
+                                   (unsigned)(w[b][1] >> 32) == seq));
+                if (all)
+                    break;
+                if (++polls >= kCoopSpin) {
+                    sh_stall = 1;
+                    break;
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                hr[b0 + b] = value_of(w[b][0], w[b][1]);
+        }
+        __syncthreads();
+        if (sh_stall || sh_stop)
+            break;
+        beta = sh_ab[1];
+        first = false;
+    }
+    if (sh_stall)
+        fs.stalled = 1;
+    if (gid == 0 && t == 0)
+        *st = fs;
+#pragma unroll
+    for (int m = 0; m < CPT; ++m)
+        if (own_bits >> m & 1) {
+            const int row = no[m] / n0, i = no[m] - row * n0;
+            const int64_t c = padded(i, row % n1, row / n1);
+            x[c] = xl[t + NT * m];
+            r[c] = rv[m];
+            pg[c] = pw[wi[m] & 0xffff];
+        }
+}
+
+// Bytes of LDS: the window, the coefficient tables, x.
+size_t coop3_lds(const Coop3Grid& c)
+{
+    return ((size_t)c.nwin + 14 + (size_t)c.nt * c.cpt) * sizeof(double);
+}
+
+// The pencils' shape: the one with the least estimate of an iteration's time
+// in us, from measured parts: an exchange of G workgroups (twice), a cell of
+// a lane per wave of a SIMD, the fixed chain, and the halo words' traffic.
+// G = 0: none fits (more than 256 pencils of 4096 cells, about 100^3).  us per
+// iteration, the streaming tiles before and this: 45 x 52 x 61 22.6 -> 8.9,
+// 64^3 22.9 -> 9.6, 96^3 30.6 -> 15.3, 100^3 32 -> 17.6.
+Coop3Grid coop3_grid(const Geo& g)
+{
+    constexpr int shape[][2] = {{256, 2}, {256, 4}, {512, 4}, {512, 8}};
+    Coop3Grid best{};
+    double cost = 1e30;
+    const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+    if (n0 > 1024)
+        return best;
+    for (int by = 1; by <= n1 && by <= 64; ++by)
+        for (int bz = 1; bz <= n2 && bz <= 64; ++bz) {
+            const int64_t cells = (int64_t)n0 * by * bz;
+            const int64_t G64 = (int64_t)((n1 + by - 1) / by) * ((n2 + bz - 1) / bz);
+            if (cells > 4096 || G64 > kCoopMaxGroups)
+                continue;
+            const int G = (int)G64;
+            int q = 0;
+            while (shape[q][0] * shape[q][1] < cells)
+                ++q;
+            const int nt = shape[q][0], cpt = shape[q][1];
+            const int halo = 2 * (by + bz) * n0;
+            Coop3Grid c{};
+            c.G = G;
+            c.by = by;
+            c.bz = bz;
+            c.gy = (n1 + by - 1) / by;
+            c.e0 = n0 + 2;
+            c.e1 = c.e0 * (by + 2);
+            c.nwin = c.e1 * (bz + 2);
+            c.nt = nt;
+            c.cpt = cpt;
+            if (halo > kCoopHalo * (nt - kWave) || c.nwin >= 1 << 16 ||
+                coop3_lds(c) > 150 * 1024)
+                continue;
+            const double us = 2.0 * (1.3 + 0.1 * std::log2((double)G) + 0.006 * G) + 1.5 +
+                              0.25 * (nt / 256) * cpt + 1e-3 * halo / (nt - kWave) * 200.0 +
+                              3.2e-6 * halo * G;
+            if (us < cost) {
+                cost = us;
+                best = c;
+            }
+        }
+    best.every = best.G > 1 && best.G <= 32 ? 8 : 1;
+    best.c00 = (int)g.idx(g.h, g.h, g.h);
+    best.px = (int)g.px;
+    best.pxy = g.px * g.py;
+    return best;
+}
+
+template <int NT, int CPT>
+const void* coop3_kernel(int G)
+{
+    return G <= kWave       ? (const void*)k_pcg_solve_coop3<NT, CPT, 1>
+           : G <= 2 * kWave ? (const void*)k_pcg_solve_coop3<NT, CPT, 2>
+                            : (const void*)k_pcg_solve_coop3<NT, CPT, 4>;
+}
+
 } // namespace
 
 bool pcg_coop_fits(const Geo& g)
 {
-    if (g.dim != 2)
-        return false;
+    if (g.dim == 3)
+        return coop3_grid(g).G > 0;
     const CoopGrid cg = coop_grid(g);
     if (cg.G > kCoopMaxGroups)
         return false;
@@ -575,6 +934,9 @@ bool pcg_coop_fits(const Geo& g)
 
 size_t coop_xch_bytes(const Geo& g)
 {
+    if (g.dim == 3)
+        return ((size_t)coop3_grid(g).G * 16 + 2 * (size_t)g.n[0] * g.n[1] * g.n[2]) *
+               sizeof(Word);
     const CoopGrid cg = coop_grid(g);
     return (size_t)cg.G * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
 }
@@ -586,7 +948,6 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
         throw CfError(CF_EINVAL, "grid does not fit the cooperative PCG");
     if (max_its < 1)
         throw CfError(CF_EINVAL, "the cooperative PCG runs at least one iteration per launch");
-    const CoopGrid cg = coop_grid(g);
     // a word is new when it carries its exchange's number: the numbers go on
     // from launch to launch, and before they wrap the buffer is cleared
     if (seq > 0xffffffffu - 2u * (unsigned)max_its - 2u) {
@@ -595,19 +956,38 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
     }
     CoopXch xc;
     xc.part = (Word*)xch;
-    xc.halo = xc.part + (size_t)cg.G * 16;
     xc.seq0 = seq;
     Geo ga = g;
-    CoopGrid cga = cg;
+    CoopGrid cg;
+    Coop3Grid c3;
     double *xa = x, *ra = r, *pa = p;
     PcgState* sta = st;
     int ma = max_its;
-    void* args[] = {&ga, &cga, &xa, &ra, &pa, &sta, &xc, &ma};
-    const void* fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
-         : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
-                       : coop_kernel<512, 8>(cg.G);
-    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(cg.G * cg.every), dim3(cg.nt), args,
-                                                    (unsigned)coop_lds(g, cg), s);
+    void* args[] = {&ga, &cg, &xa, &ra, &pa, &sta, &xc, &ma};
+    const void* fn;
+    dim3 grid, block;
+    size_t lds;
+    if (g.dim == 3) {
+        c3 = coop3_grid(g);
+        args[1] = &c3;
+        xc.halo = xc.part + (size_t)c3.G * 16;
+        fn = c3.nt == 256 ? (c3.cpt == 2 ? coop3_kernel<256, 2>(c3.G) : coop3_kernel<256, 4>(c3.G))
+             : c3.cpt == 4 ? coop3_kernel<512, 4>(c3.G)
+                           : coop3_kernel<512, 8>(c3.G);
+        grid = dim3(c3.G * c3.every);
+        block = dim3(c3.nt);
+        lds = coop3_lds(c3);
+    } else {
+        cg = coop_grid(g);
+        xc.halo = xc.part + (size_t)cg.G * 16;
+        fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
+             : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
+                           : coop_kernel<512, 8>(cg.G);
+        grid = dim3(cg.G * cg.every);
+        block = dim3(cg.nt);
+        lds = coop_lds(g, cg);
+    }
+    const hipError_t e = hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
     if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
         (void)hipGetLastError(); // refused before anything ran
         return false;
