@@ -68,14 +68,11 @@ __device__ __forceinline__ void dd_norm(double& hi, double& lo)
 
 // ---- B-spline sampling (Cajita SplineData / evaluateSpline / G2P::value,
 // called at src/Interpolation.hpp:30-41) -------------------------------------
+// Weights at the fraction t of a logical coordinate.
 template <int ORDER>
-__device__ __forceinline__ void spline_weights(double xi, int& s0,
-                                               double (&w)[ORDER + 1])
+__device__ __forceinline__ void spline_of(double t, double (&w)[ORDER + 1])
 {
-    int fl = (int)xi;
-    double t = xi - (double)fl;
     if constexpr (ORDER == 1) {
-        s0 = fl;
         w[0] = 1.0 - t;
         w[1] = t;
     } else {
@@ -83,12 +80,19 @@ __device__ __forceinline__ void spline_weights(double xi, int& s0,
         double omt = 1.0 - t;
         double t2 = t * t;
         double t3 = t2 * t;
-        s0 = fl - 1;
         w[0] = ((omt * omt) * omt) * c16;
         w[1] = ((3.0 * t3 - 6.0 * t2) + 4.0) * c16;
         w[2] = (((-3.0 * t3 + 3.0 * t2) + 3.0 * t) + 1.0) * c16;
         w[3] = t3 * c16;
     }
+}
+template <int ORDER>
+__device__ __forceinline__ void spline_weights(double xi, int& s0,
+                                               double (&w)[ORDER + 1])
+{
+    int fl = (int)xi;
+    s0 = ORDER == 1 ? fl : fl - 1;
+    spline_of<ORDER>(xi - (double)fl, w);
 }
 
 // Logical coordinate along axis d, clamped so the stencil stays inside the

@@ -1,6 +1,6 @@
 // cf_kernels.hip -- HIP kernels of the CajitaFluids hot path for gfx950:
-// advection, inputs, ghost fill, divergence and projection.  The PCG lives
-// in cf_pcg.hip; the streaming-kernel building blocks in cf_stream.hpp.
+// inputs, ghost fill, divergence and projection.  Advection lives in
+// cf_advect.hip, the PCG in cf_pcg.hip; the streaming-kernel building blocks in cf_stream.hpp.
 #include <hip/hip_runtime.h>
 
 #include "cf_stream.hpp"
@@ -8,83 +8,11 @@
 namespace cfmi
 {
 
-// ---- advection: TimeIntegrator::advect for every entity in one launch ------
-// (src/TimeIntegrator.hpp:81-116): each lane owns one (i, j, k) of the union
-// of the owned boxes and advects every entity owning that index.
-//
-// Occupancy: the 3-D kernels with linear velocity sampling keep the 64
-// cubic taps of a field sample in flight and would take 146 VGPRs (3 waves
-// per SIMD); capping them at 128 VGPRs (4 waves, a 36-byte spill) runs the
-// 256^3 vortex tank's advection in 3.0 ms instead of 4.15 (64 x 4 x 1
-// blocks).  Higher caps spill more than they gain (5 waves: 4.2 ms, 6:
-// 5.2 ms).
-template <int DIM, int VORDER>
-constexpr int advect_min_waves()
-{
-    return DIM == 3 && VORDER == 1 ? 4 : 1;
-}
-
-template <int DIM, int FORDER, int VORDER>
-__global__ __launch_bounds__(256, (advect_min_waves<DIM, VORDER>())) void k_advect(Geo g,
-                                                                                 Fields cur,
-                                                                                 Fields next)
-{
-    const int i = g.h + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = g.h + blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = g.own_lo(2) + blockIdx.z * blockDim.z + threadIdx.z;
-    const int l[3] = {i, j, k};
-    const double* u = cur.e[1];
-    const double* v = cur.e[2];
-    const double* w = cur.e[3];
-#pragma unroll
-    for (int e = 0; e <= DIM; ++e) {
-        bool own = true;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            own = own && l[d] < g.own_hi[e][d];
-        if (!own)
-            continue;
-        double x0[3] = {0, 0, 0}, tr[3];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d)
-            x0[d] = coord(g, e, d, l[d]);
-        rk3<DIM, VORDER>(g, u, v, w, x0, tr);
-        next.e[e][g.idx(i, j, k)] =
-            interpolate<DIM, FORDER>(g, e, cur.e[e], tr);
-    }
-}
-
 static dim3 union_grid(const Geo& g, dim3 blk)
 {
     const int ex = g.uni_hi[0] - g.h, ey = g.uni_hi[1] - g.h;
     const int ez = g.dim == 3 ? g.uni_hi[2] - g.h : 1;
     return dim3((ex + blk.x - 1) / blk.x, (ey + blk.y - 1) / blk.y, (ez + blk.z - 1) / blk.z);
-}
-
-// 3-D blocks of 32 x 4 x 2 points: two z planes share the cubic stencils in
-// the CU's caches (2.88 against 3.0 ms for 64 x 4 x 1 at 256^3).
-template <int DIM, int FORDER, int VORDER>
-static void advect_t(const Geo& g, Fields cur, Fields next, hipStream_t s)
-{
-    const dim3 blk = DIM == 3 ? dim3(32, 4, 2) : dim3(64, 4, 1);
-    hipLaunchKernelGGL((k_advect<DIM, FORDER, VORDER>), union_grid(g, blk), blk,
-                       0, s, g, cur, next);
-}
-
-void launch_advect(const Geo& g, Fields cur, Fields next, hipStream_t s)
-{
-    const int key = g.dim * 100 + g.field_order * 10 + g.vel_order;
-    switch (key) {
-    case 211: advect_t<2, 1, 1>(g, cur, next, s); break;
-    case 231: advect_t<2, 3, 1>(g, cur, next, s); break;
-    case 213: advect_t<2, 1, 3>(g, cur, next, s); break;
-    case 233: advect_t<2, 3, 3>(g, cur, next, s); break;
-    case 311: advect_t<3, 1, 1>(g, cur, next, s); break;
-    case 331: advect_t<3, 3, 1>(g, cur, next, s); break;
-    case 313: advect_t<3, 1, 3>(g, cur, next, s); break;
-    case 333: advect_t<3, 3, 3>(g, cur, next, s); break;
-    default: break;
-    }
 }
 
 // ---- inputs: Solver::_addInputs (src/Solver.hpp:181-263) -----------------

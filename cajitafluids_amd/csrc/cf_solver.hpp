@@ -78,7 +78,7 @@ enum TimedKernel
     TK_ADVECT = 6,
     TK_RESIDUAL = 7,   // FP64 defect-correction residual
     TK_VCYCLE = 8,     // one multigrid V-cycle
-    TK_PCG_COOP = 9,   // one launch of the cooperative 2-D PCG
+    TK_PCG_COOP = 9,   // one launch of the cooperative PCG
     TK_COUNT = 10
 };
 
@@ -187,7 +187,7 @@ class VelocityCorrector
     int runIterations(T* x, T* r, DevArray<T> (&p)[2], int& cur, int predict,
                       int tk0);
     int runPcg64(const double* b, double* x, double tol, int maxit);
-    // the whole FP64 solve by the cooperative 2-D kernel (pcg_coop_fits)
+    // the whole FP64 solve by the cooperative kernel (pcg_coop_fits)
     int runCoop(double* x);
     void readState(PcgState& host);
     void readRefine();
@@ -202,7 +202,7 @@ class VelocityCorrector
     DevArray<double> _lhs, _rhs, _r, _p[2];
     DevArray<float> _d32, _r32, _p32[2];
     DevArray<double> _red_partials, _scratch;
-    DevArray<double> _xch; // exchange buffer of the cooperative 2-D PCG
+    DevArray<double> _xch; // exchange buffer of the cooperative PCG
     unsigned _xch_seq = 0; // the last exchange number used in it
     bool _coop_off = false; // the runtime refused a cooperative launch
     DevArray<unsigned> _red_counter;
