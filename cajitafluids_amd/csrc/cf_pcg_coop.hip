@@ -20,7 +20,8 @@
 //   - each of an iteration's two reductions: a workgroup reduction, then the
 //     workgroup's double-double partial published and every workgroup's
 //     partials read and summed in one fixed order, so that every workgroup
-//     holds the same alpha, beta and stop decision.
+//     holds the same alpha, beta and stop decision.  A wave of its own, with
+//     no cells, does this part and the scalars (coop_scalars).
 //
 // What bounds it is the two exchanges' latency: a value travels as 64-bit
 // words of 32 bits of it and the exchange's sequence number, stored and
@@ -32,7 +33,13 @@
 // words, 1.9 us with the wave sums by lane moves instead of LDS permutes,
 // 1.65 us with the workgroups on one XCD (every eighth block of the launch,
 // while that many fit the GPU; the others return at once, and nothing but
-// the latency depends on where the blocks really run).
+// the latency depends on where the blocks really run).  Polling the XCD's own
+// L2 (with an invalidate or an atomic a poll) was no faster than agent scope.
+//
+// Beside them, a strip's own chain, 2.9 -> 2.0 us of an iteration: sums whose
+// steps wait for one addition (dd_merge), r.r and r.z summed in alternate
+// lanes, the stop test's root and division beside the next direction, halo
+// cells kept as D^-1 r, and no halo work where no strip is next.
 //
 // Every value is the streaming kernels' expression on the same operands, so
 // x, r, the direction and the state come out with the same bits.  A poll
@@ -54,6 +61,7 @@ namespace
 {
 
 constexpr int kCoopMaxGroups = 256;
+constexpr int kCoopCells = 4096; // of a strip or pencil at most
 constexpr unsigned kCoopSpin = 1u << 22; // polls (about 1 us each) before a wait counts as stalled
 
 // Strip layout: R rows per strip, G strips; window row pitch e0 = n0 + 2
@@ -69,21 +77,24 @@ struct CoopGrid
 };
 
 // The strips' shape: 4 cells a lane of 256 lanes while that makes at most 64
-// strips (one partial a lane of the gather), 4 of 512 up to 128 strips (two a
-// lane), else 8 of 512.  Fewer, larger strips shorten the exchanges and
-// lengthen the strip's own chain.  us per iteration at (256, 4), (512, 4),
-// (512, 8): 32^2 2.9 (one strip), 3.8, 5.0; 128^2 5.7, 5.8, 6.7; 256^2 6.8,
-// 7.7, 8.4; 391 x 263 9.7, 7.7, 9.0; 512^2 13.4, 9.1, 9.4; 700 x 500 -, 14.9,
-// 10.5; 1024^2 -, -, 16.9 (the streaming kernels 32.2).  1024 lanes, and 2
-// cells a lane, were slower or within 2% everywhere.
+// strips, 4 of 512 up to 128 strips, else 10 of 448 (with the scalars' wave two
+// waves a SIMD: 8 of 512 with it left 168 registers a lane, and spilled).
+// Fewer, larger strips shorten the exchanges and lengthen the strip's own
+// chain.  us per iteration at 4 of 256, 4 of 512 and 8 of 512 lanes, with the
+// scalars in a wave of cells: 32^2 2.9 (one strip), 3.8, 5.0; 128^2 5.7, 5.8,
+// 6.7; 256^2 6.8, 7.7, 8.4; 391 x 263 9.7, 7.7, 9.0; 512^2 13.4, 9.1, 9.4;
+// 700 x 500 -, 14.9, 10.5; 1024^2 -, -, 16.9.  Now, at the shape chosen: 32^2
+// 2.0, 128^2 4.3, 256^2 5.6, 391 x 263 6.2, 512^2 7.1, 700 x 500 9.0, 1024^2
+// 14.7 (the streaming kernels 32.2).  1024 lanes, and 2 cells a lane, were
+// slower or within 2% everywhere.
 CoopGrid coop_grid(const Geo& g)
 {
-    constexpr int shape[3][3] = {{256, 4, 64}, {512, 4, 128}, {512, 8, kCoopMaxGroups}};
+    constexpr int shape[3][3] = {{256, 4, 64}, {512, 4, 128}, {448, 10, kCoopMaxGroups}};
     CoopGrid cg;
     for (const auto& sh : shape) {
         cg.nt = sh[0];
         cg.cpt = sh[1];
-        cg.R = cg.nt * cg.cpt / g.n[0];
+        cg.R = (cg.nt * cg.cpt < kCoopCells ? cg.nt * cg.cpt : kCoopCells) / g.n[0];
         if (cg.R > g.n[1])
             cg.R = g.n[1];
         cg.G = cg.R > 0 ? (g.n[1] + cg.R - 1) / cg.R : INT_MAX;
@@ -155,145 +166,263 @@ __device__ __forceinline__ double move_half(double v)
     }
 }
 
-// Sums NV double-double values over groups of `width` lanes (a power of two),
-// the result in each of them.
-template <int NV>
-__device__ __forceinline__ void wave_sum(double (&hi)[NV], double (&lo)[NV], int width)
+// (hi, lo) += (oh, ol): the high parts' rounding error goes to the low part,
+// which is summed as it is (as in dd_acc_prod): one addition a step is on the
+// high parts' chain instead of dd_add's seven.
+__device__ __forceinline__ void dd_merge(double& hi, double& lo, double oh, double ol)
 {
-#define CF_STEP(W, MOVE)                                  \
-    if (width > W) {                                      \
-        _Pragma("unroll") for (int v = 0; v < NV; ++v)    \
-        {                                                 \
-            const double oh = MOVE(hi[v]), ol = MOVE(lo[v]); \
-            dd_add(hi[v], lo[v], oh, ol);                 \
-        }                                                 \
+    const double s = hi + oh;
+    const double t = s - hi;
+    const double e = (hi - (s - t)) + (oh - t);
+    lo = (lo + ol) + e;
+    hi = s;
+}
+#define CF_STEP(MOVE)                                   \
+    {                                                   \
+        const double oh = MOVE(h), ol = MOVE(l);        \
+        dd_merge(h, l, oh, ol);                         \
     }
-    CF_STEP(1, move_row<0xB1>)  // quad_perm 1 0 3 2
-    CF_STEP(2, move_row<0x4E>)  // quad_perm 2 3 0 1
-    CF_STEP(4, move_row<0x141>) // row_half_mirror
-    CF_STEP(8, move_row<0x140>) // row_mirror
-    CF_STEP(16, move_half<16>)
-    CF_STEP(32, move_half<32>)
+
+// Sum of (h, l) over groups of `width` lanes (a power of two), in each of them.
+__device__ __forceinline__ void wave_sum(double& h, double& l, int width)
+{
+    if (width > 1)
+        CF_STEP(move_row<0xB1>) // quad_perm 1 0 3 2
+    if (width > 2)
+        CF_STEP(move_row<0x4E>) // quad_perm 2 3 0 1
+    if (width > 4)
+        CF_STEP(move_row<0x141>) // row_half_mirror
+    if (width > 8)
+        CF_STEP(move_row<0x140>) // row_mirror
+    if (width > 16)
+        CF_STEP(move_half<16>)
+    if (width > 32)
+        CF_STEP(move_half<32>)
+}
+// The sums over the even lanes and over the odd lanes, in each even and each
+// odd lane, of values that repeat every `width` lanes or (width >= 16) are
+// zero past them.  As in wave_sum, the two lanes of a step add the same two
+// pairs, so every lane ends with the same (h, l) bits: the words of a
+// published partial come from different lanes.
+__device__ __forceinline__ void pair_sum(double& h, double& l, int width)
+{
+    CF_STEP(move_row<0x4E>)
+    if (width > 8)
+        CF_STEP(move_row<0x128>) // row_ror 8
+    if (width > 4)
+        CF_STEP(move_row<0x124>) // row_ror 4
+    if (width > 16)
+        CF_STEP(move_half<16>)
+    if (width > 32)
+        CF_STEP(move_half<32>)
+}
 #undef CF_STEP
-}
 
-// One reduction of the strip's lanes' NV sums over all strips: the workgroup
-// sum, its publication, and in wave 0 the rounded totals.  Wave 0 returns
-// with out set; the other waves return after the workgroup's barrier.
-// PPL: strips per lane of wave 0's gather.
-// shadow(): work that every wave does while the words travel.
-template <int NT, int NV, int PPL, class F>
-__device__ __forceinline__ void coop_reduce(double (&hi)[NV], double (&lo)[NV], int gid, int G,
-                                            Word* part, int off, unsigned seq,
-                                            double (*red)[2][NT / kWave], int* stall,
-                                            double (&out)[NV], F&& shadow)
+// What the waves of a workgroup share.  A workgroup is NW waves of cells and
+// one wave of scalars (coop_scalars): the cells' waves leave their wave sums
+// in red, the scalars' wave forms the totals over all workgroups.
+template <int NW>
+struct CoopShared
 {
-    constexpr int NW = NT / kWave;
-    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-        dd_norm(hi[v], lo[v]);
-    wave_sum<NV>(hi, lo, kWave);
-    if (lane == 0) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            red[v][0][wv] = hi[v];
-            red[v][1][wv] = lo[v];
-        }
-    }
-    __syncthreads();
-    if (wv != 0) {
-        shadow();
-        return;
-    }
-    double h[NV], l[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        h[v] = red[v][0][lane & (NW - 1)];
-        l[v] = red[v][1][lane & (NW - 1)];
-    }
-    wave_sum<NV>(h, l, NW);
-    if (G > 1) {
-        if (lane < 4 * NV) { // word lane & 3 of value lane >> 2
-            const double a = NV > 1 && lane >= 4 ? h[NV - 1] : h[0];
-            const double b = NV > 1 && lane >= 4 ? l[NV - 1] : l[0];
-            const double v = lane & 2 ? b : a;
-            put_word(part + (size_t)gid * 16 + off + lane, seq,
-                     (unsigned)(lane & 1 ? __double2hiint(v) : __double2loint(v)));
-        }
-        shadow();
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-            h[v] = l[v] = 0.0;
-        Word w[PPL][4 * NV];
-        unsigned polls = 0;
-        for (;;) {
-            bool all = true;
-#pragma unroll
-            for (int u = 0; u < PPL; ++u) {
-                const int q = lane + kWave * u;
-                const Word* pq = part + (size_t)(q < G ? q : 0) * 16 + off;
-#pragma unroll
-                for (int k = 0; k < 4 * NV; ++k)
-                    w[u][k] = get_word(pq + k);
-            }
-#pragma unroll
-            for (int u = 0; u < PPL; ++u)
-#pragma unroll
-                for (int k = 0; k < 4 * NV; ++k)
-                    all = all && (unsigned)(w[u][k] >> 32) == seq;
-            if (__all(all))
-                break;
-            if (++polls >= kCoopSpin) {
-                if (lane == 0)
-                    *stall = 1;
-                break;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < PPL; ++u)
-            if (lane + kWave * u < G) {
-#pragma unroll
-                for (int v = 0; v < NV; ++v)
-                    dd_add(h[v], l[v], value_of(w[u][4 * v], w[u][4 * v + 1]),
-                           value_of(w[u][4 * v + 2], w[u][4 * v + 3]));
-            }
-        wave_sum<NV>(h, l, G < kWave ? 1 << (32 - __builtin_clz(G - 1)) : kWave);
-    } else {
-        shadow();
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-        out[v] = h[v] + l[v];
-}
+    static constexpr int N = NW <= 4 ? 4 : 8; // NW rounded up, zeros past NW
+    double pq[2][N];    // p.q of the waves, high and low parts
+    double rr[2][2][N]; // r.r, r.z
+    double alpha, beta;
+    int stop, stall;
 
-// Bits of a lane's cell slots: owned (a slot past the strip's last cell is
-// not, and carries the first cell's window index; its stores and sums are
-// masked), and in the strip's top / bottom row.
-struct CoopSlots
-{
-    unsigned own, top, bottom;
+    // before the workgroup's first barrier
+    __device__ __forceinline__ void clear(int t)
+    {
+        if (t < 2 * N)
+            pq[t / N][t % N] = 0.0;
+        if (t < 4 * N)
+            rr[t / N / 2][t / N % 2][t % N] = 0.0;
+        if (t == 0)
+            stop = stall = 0;
+    }
 };
 
-template <int NT, int CPT, int PPL>
-__global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, double* __restrict__ x,
-                                                       double* __restrict__ r,
-                                                       double* __restrict__ pg, PcgState* st,
-                                                       CoopXch xc, int max_its)
+// A wave's sum of (h, l) for the scalars' wave; the sums of (h0, l0) and of
+// (h1, l1), the first exchange handing each lane one of the two.
+template <int NW>
+__device__ __forceinline__ void leave_pq(CoopShared<NW>& sh, double h, double l)
+{
+    wave_sum(h, l, kWave);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        sh.pq[0][threadIdx.x / kWave] = h;
+        sh.pq[1][threadIdx.x / kWave] = l;
+    }
+}
+template <int NW>
+__device__ __forceinline__ void leave_rr(CoopShared<NW>& sh, const double (&hi)[2],
+                                         const double (&lo)[2])
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool odd = lane & 1;
+    double h = odd ? hi[1] : hi[0], l = odd ? lo[1] : lo[0];
+    const double oh = move_row<0xB1>(odd ? hi[0] : hi[1]), ol = move_row<0xB1>(odd ? lo[0] : lo[1]);
+    dd_merge(h, l, oh, ol);
+    pair_sum(h, l, kWave);
+    if (lane < 2) {
+        sh.rr[lane][0][threadIdx.x / kWave] = h;
+        sh.rr[lane][1][threadIdx.x / kWave] = l;
+    }
+}
+
+// Polls the four words at each of `at` until all carry seq; false: stalled.
+// With one place a lane, only the lanes that want theirs read (of up to 32
+// workgroups most have none: 128^2 4.8 -> 4.4 us an iteration); with more, a
+// branch for each costs more than the reads it saves (512^2 7.1 -> 8.3).
+template <int N>
+__device__ __forceinline__ bool poll_words(const Word* const (&at)[N], const bool (&want)[N],
+                                           unsigned seq, Word (&w)[N][4])
+{
+    for (unsigned polls = 0; polls < kCoopSpin; ++polls) {
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            if (N > 1 || want[u]) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    w[u][k] = get_word(at[u] + k);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    all = all && (unsigned)(w[u][k] >> 32) == seq;
+            }
+        if (__all(all))
+            return true;
+    }
+    return false;
+}
+
+// The scalars' wave: per iteration p.q's total and alpha, then r.r's and
+// r.z's and beta; it keeps the PCG state (the same in every workgroup) in its
+// first lane.  The stop test's square root and division run beside the cells'
+// next direction and stencil, so a stop is seen one direction later.  The
+// barriers are the cells' waves' (A, after periodic x's copies again, B, C,
+// D, E).  PQ: strips per lane of the gather of the two sums (32 lanes each).
+template <int NW, int PQ>
+__device__ __forceinline__ void coop_scalars(CoopShared<NW>& sh, PcgState& fs, int gid, int G,
+                                             const CoopXch& xc, bool periodic_x, int max_its)
+{
+    constexpr int N = CoopShared<NW>::N;
+    constexpr int P1 = PQ > 1 ? PQ / 2 : 1; // strips per lane of p.q's gather
+    const int lane = threadIdx.x & (kWave - 1);
+    unsigned seq = xc.seq0;
+    double rr = 0.0, rz = 0.0;
+    const int width = G <= 1 ? 1 : G < kWave ? 1 << (32 - __builtin_clz(G - 1)) : kWave;
+    for (int its = 1;; ++its) {
+        __syncthreads(); // A
+        if (periodic_x)
+            __syncthreads();
+        if (its > 1 && lane == 0) {
+            finish_update(&fs, rr, rz);
+            sh.stop = fs.done;
+        }
+        __syncthreads(); // B
+        if (sh.stop)
+            break;
+        double h = sh.pq[0][lane & (N - 1)], l = sh.pq[1][lane & (N - 1)];
+        wave_sum(h, l, N);
+        ++seq;
+        if (G > 1) {
+            if (lane < 4) {
+                const double v = lane & 2 ? l : h;
+                put_word(xc.part + (size_t)gid * 16 + lane, seq,
+                         (unsigned)(lane & 1 ? __double2hiint(v) : __double2loint(v)));
+            }
+            const Word* at[P1];
+            bool want[P1];
+            Word w[P1][4];
+#pragma unroll
+            for (int u = 0; u < P1; ++u) {
+                const int q = lane + kWave * u;
+                want[u] = q < G;
+                at[u] = xc.part + (size_t)(q < G ? q : 0) * 16;
+            }
+            if (!poll_words<P1>(at, want, seq, w) && lane == 0)
+                sh.stall = 1;
+            h = l = 0.0;
+#pragma unroll
+            for (int u = 0; u < P1; ++u)
+                if (want[u])
+                    dd_merge(h, l, value_of(w[u][0], w[u][1]), value_of(w[u][2], w[u][3]));
+            wave_sum(h, l, width);
+        }
+        if (lane == 0) {
+            fs.alpha = fs.rho / (h + l);
+            sh.alpha = fs.alpha;
+        }
+        __syncthreads(); // C
+        if (sh.stall)
+            break;
+        __syncthreads(); // D
+        // r.r in the even lanes, r.z in the odd ones
+        const int v = lane & 1, wv = lane >> 1 & (N - 1);
+        h = sh.rr[v][0][wv];
+        l = sh.rr[v][1][wv];
+        pair_sum(h, l, 2 * N);
+        ++seq;
+        if (G > 1) {
+            if (lane < 8) {
+                const int k = lane >> 1;
+                const double d = k & 2 ? l : h;
+                put_word(xc.part + (size_t)gid * 16 + 8 + 4 * v + k, seq,
+                         (unsigned)(k & 1 ? __double2hiint(d) : __double2loint(d)));
+            }
+            const Word* at[PQ];
+            bool want[PQ];
+            Word w[PQ][4];
+#pragma unroll
+            for (int u = 0; u < PQ; ++u) {
+                const int q = (lane >> 1) + kWave / 2 * u;
+                want[u] = q < G;
+                at[u] = xc.part + (size_t)(q < G ? q : 0) * 16 + 8 + 4 * v;
+            }
+            if (!poll_words<PQ>(at, want, seq, w) && lane == 0)
+                sh.stall = 1;
+            h = l = 0.0;
+#pragma unroll
+            for (int u = 0; u < PQ; ++u)
+                if (want[u])
+                    dd_merge(h, l, value_of(w[u][0], w[u][1]), value_of(w[u][2], w[u][3]));
+            pair_sum(h, l, width < 8 ? 16 : 2 * width);
+        }
+        rr = h + l;
+        rz = move_row<0xB1>(rr);
+        if (lane == 0)
+            sh.beta = rz / fs.rho;
+        __syncthreads(); // E
+        if (sh.stall)
+            break;
+        if (its >= max_its) {
+            if (lane == 0)
+                finish_update(&fs, rr, rz);
+            break;
+        }
+    }
+}
+
+template <int NT, int CPT, int PQ>
+__global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop(Geo g, CoopGrid cg,
+                                                               double* __restrict__ x,
+                                                               double* __restrict__ r,
+                                                               double* __restrict__ pg,
+                                                               PcgState* st, CoopXch xc,
+                                                               int max_its)
 {
     if (blockIdx.x % cg.every)
         return;
+    constexpr int NW = NT / kWave;
     extern __shared__ double lds[];
     double* pw = lds;             // the direction window
     double* tab = lds + cg.nwin;  // diag[0..6], then dinv[0..6]
-    double* hr = tab + 14;        // halo rows' r [2][n0]
-    double* hd = hr + 2 * g.n[0]; // and their D^-1
-    __shared__ double red[2][2][NT / kWave];
-    __shared__ double sh_ab[2]; // alpha, beta
-    __shared__ int sh_stop, sh_stall;
-    // The state is read once, here; thread 0 of every workgroup keeps the same
-    // copy in registers, and workgroup 0 stores it back at the end.  A read
-    // of *st after a write in this kernel could be served by the scalar
+    double* hz = tab + 14;        // halo rows' D^-1 r [2][n0]
+    double* hd = hz + 2 * g.n[0]; // and their D^-1
+    __shared__ CoopShared<NW> sh;
+    // The state is read once, here; the scalars' wave of every workgroup keeps
+    // the same copy in registers, and workgroup 0 stores it back at the end.
+    // A read of *st after a write in this kernel could be served by the scalar
     // cache, which vector stores do not update.
     PcgState fs = *st;
     const int t = threadIdx.x;
@@ -301,11 +430,11 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
     const int n0 = g.n[0], n1 = g.n[1], e0 = cg.e0;
     const int j0 = gid * cg.R;
     const int nrows = (j0 + cg.R < n1 ? cg.R : n1 - j0);
+    const int ncell = nrows * n0;
     const double s = offdiag<double>(g);
     const double ring0 = copysign(0.0, s);
-    if (t == 0)
-        sh_stall = 0;
-    for (int e = t; e < cg.nwin; e += NT)
+    sh.clear(t);
+    for (int e = t; e < cg.nwin; e += NT + kWave)
         pw[e] = ring0;
 #pragma unroll
     for (int q = 0; q < 7; ++q)
@@ -316,6 +445,16 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
     __syncthreads();
     if (fs.done)
         return;
+    if (__builtin_amdgcn_readfirstlane(t / kWave) == NW) {
+        __syncthreads(); // the cells are loaded
+        coop_scalars<NW, PQ>(sh, fs, gid, G, xc, g.periodic[0], max_its);
+        if (gid == 0 && t == NT) {
+            if (sh.stall)
+                fs.stalled = 1;
+            *st = fs;
+        }
+        return;
+    }
     bool first = fs.iter == 0;
     double beta = fs.beta;
 
@@ -336,39 +475,37 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
         const int side = e >= n0 ? 1 : 0, i = e - side * n0;
         if (side == 0 ? has_top : has_bot) {
             const int64_t c = cg.c00 + i + (int64_t)cg.px * (side == 0 ? jtop : jbot);
-            hr[e] = r[c];
             hd[e] = tab[7 + cell_cnt(i, side == 0 ? jtop : jbot)];
+            hz[e] = hd[e] * r[c];
             if (!first)
                 pw[halo_at(side, i)] = pg[c];
         }
     }
 
+    // Slots past the strip's last cell carry the first cell's window index;
+    // their stores and sums are masked.
     int wi[CPT]; // window indices
-    double rv[CPT], qv[CPT], xv[CPT], dg[CPT], dv[CPT];
-    CoopSlots sl{0, 0, 0};
+    bool own[CPT];
+    double rv[CPT], qv[CPT], xv[CPT], dg[CPT], dv[CPT], pn[CPT];
 #pragma unroll
     for (int m = 0; m < CPT; ++m) {
         const int L = t + NT * m;
         const int i = L % n0, jj = L / n0;
+        own[m] = L < ncell;
         wi[m] = 1 + e0; // strip cell (0, 0)
-        rv[m] = 0.0;
-        qv[m] = 0.0;
-        xv[m] = 0.0;
+        rv[m] = qv[m] = xv[m] = pn[m] = 0.0;
         dg[m] = tab[0];
         dv[m] = tab[7];
-        if (jj < nrows) {
+        if (own[m]) {
             const int cnt = cell_cnt(i, j0 + jj);
             wi[m] = (i + 1) + e0 * (jj + 1);
             dg[m] = tab[cnt];
             dv[m] = tab[7 + cnt];
-            sl.own |= 1u << m;
-            sl.top |= jj == 0 ? 1u << m : 0u;
-            sl.bottom |= jj == nrows - 1 ? 1u << m : 0u;
             const int64_t c = cg.c00 + i + (int64_t)cg.px * (j0 + jj);
             rv[m] = r[c];
             xv[m] = x[c];
             if (!first)
-                pw[wi[m]] = pg[c];
+                pn[m] = pg[c];
         }
     }
     // padded index of a slot's cell
@@ -381,10 +518,6 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
     for (int its = 1;; ++its) {
         // direction: p = D^-1 r, or fma(beta, p, D^-1 r), for the strip's
         // cells and its halo rows
-        double pn[CPT];
-#pragma unroll
-        for (int m = 0; m < CPT; ++m)
-            pn[m] = pw[wi[m]];
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const double z = dv[m] * rv[m];
@@ -392,17 +525,17 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
         }
 #pragma unroll
         for (int m = 0; m < CPT; ++m)
-            if (sl.own >> m & 1)
+            if (own[m])
                 pw[wi[m]] = pn[m];
-        for (int e = t; e < 2 * n0; e += NT) {
-            const int side = e >= n0 ? 1 : 0, i = e - side * n0;
-            if (side == 0 ? has_top : has_bot) {
-                const double z = hd[e] * hr[e];
-                double* pp = pw + halo_at(side, i);
-                *pp = first ? z : fma(beta, *pp, z);
+        if (has_top || has_bot)
+            for (int e = t; e < 2 * n0; e += NT) {
+                const int side = e >= n0 ? 1 : 0, i = e - side * n0;
+                if (side == 0 ? has_top : has_bot) {
+                    double* pp = pw + halo_at(side, i);
+                    *pp = first ? hz[e] : fma(beta, *pp, hz[e]);
+                }
             }
-        }
-        __syncthreads();
+        __syncthreads(); // A
         if (g.periodic[0]) {
             for (int jw = t; jw < nrows + 2; jw += NT) {
                 double* row = pw + e0 * jw;
@@ -412,95 +545,84 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
             __syncthreads();
         }
         // q = A p in the stencil order {0}, -x, +x, -y, +y; p.q
-        double h1[1] = {0.0}, l1[1] = {0.0};
+        double h1 = 0.0, l1 = 0.0;
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const double* pp = pw + wi[m];
-            const bool own = sl.own >> m & 1;
-            const double pc = own ? pn[m] : 0.0;
+            const double pc = own[m] ? pn[m] : 0.0;
             double y = dg[m] * pn[m];
             y = fma(s, pp[-1], y);
             y = fma(s, pp[1], y);
             y = fma(s, pp[-e0], y);
             y = fma(s, pp[e0], y);
-            qv[m] = own ? y : 0.0;
-            dd_acc_prod(h1[0], l1[0], pc, qv[m]);
+            qv[m] = own[m] ? y : 0.0;
+            dd_acc_prod(h1, l1, pc, qv[m]);
         }
-        {
-            double pq[1];
-            coop_reduce<NT, 1, PPL>(h1, l1, gid, G, xc.part, 0, ++seq, red, &sh_stall, pq, [] {});
-            if (t == 0) {
-                fs.alpha = fs.rho / pq[0];
-                sh_ab[0] = fs.alpha;
-            }
-        }
-        __syncthreads();
-        if (sh_stall)
+        leave_pq(sh, h1, l1);
+        __syncthreads(); // B
+        if (sh.stop)
             break;
-        const double alpha = sh_ab[0];
+        ++seq;
+        __syncthreads(); // C
+        if (sh.stall)
+            break;
+        const double alpha = sh.alpha;
         // x = fma(alpha, p, x); r = fma(-alpha, q, r); r.r and r.(D^-1 r).
         // Past the strip's last cell q = r = 0, so rn = 0 and the sums are
         // unchanged.
-        double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
         ++seq;
 #pragma unroll
         for (int m = 0; m < CPT; ++m)
             rv[m] = fma(-alpha, qv[m], rv[m]);
         // boundary rows' new r for the neighbour strips (the one strip of a
-        // periodic axis is its own)
-        if (sl.top | sl.bottom) {
+        // periodic axis is its own), before the partials: sent with them (after
+        // D) they held up each other, 128^2 4.9 -> 5.3 us, 64^3 8.2 -> 9.2
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            if (!(side == 0 ? has_top : has_bot))
+                continue;
+            const int lo = side == 0 ? 0 : ncell - n0;
 #pragma unroll
             for (int m = 0; m < CPT; ++m) {
-                const unsigned side2 = (sl.top >> m & 1) | (sl.bottom >> m & 1) << 1;
-                if (!side2)
+                if (NT * m >= lo + n0 || NT * (m + 1) <= lo)
                     continue;
-#pragma unroll
-                for (int side = 0; side < 2; ++side) {
-                    if (!(side2 >> side & 1))
-                        continue;
-                    const int i = wi[m] - 1 - e0 * (side == 0 ? 1 : nrows);
-                    if (G > 1) {
-                        Word* hb = xc.halo + (((size_t)gid * 2 + side) * n0 + i) * 2;
-                        put_word(hb, seq, (unsigned)__double2loint(rv[m]));
-                        put_word(hb + 1, seq, (unsigned)__double2hiint(rv[m]));
-                    } else {
-                        hr[(side ^ 1) * n0 + i] = rv[m];
-                    }
+                const int i = t + NT * m - lo;
+                if (i < 0 || i >= n0)
+                    continue;
+                if (G > 1) {
+                    Word* hb = xc.halo + (((size_t)gid * 2 + side) * n0 + i) * 2;
+                    put_word(hb, seq, (unsigned)__double2loint(rv[m]));
+                    put_word(hb + 1, seq, (unsigned)__double2hiint(rv[m]));
+                } else {
+                    const int e = (side ^ 1) * n0 + i;
+                    hz[e] = hd[e] * rv[m];
                 }
             }
         }
+        double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const double z = dv[m] * rv[m];
             dd_acc_prod(hi[0], lo[0], rv[m], rv[m]);
             dd_acc_prod(hi[1], lo[1], rv[m], z);
         }
-        {
-            double rr[2];
-            coop_reduce<NT, 2, PPL>(hi, lo, gid, G, xc.part, 8, seq, red, &sh_stall, rr, [&] {
+        leave_rr(sh, hi, lo);
+        __syncthreads(); // D
 #pragma unroll
-                for (int m = 0; m < CPT; ++m)
-                    xv[m] = fma(alpha, pn[m], xv[m]);
-            });
-            if (t == 0) {
-                finish_update(&fs, rr[0], rr[1]);
-                sh_stop = fs.done || its >= max_its;
-                sh_ab[1] = fs.beta;
-            }
-        }
-        if (G > 1 && t >= kWave) {
-            // the other waves: the neighbours' boundary rows, a few cells a
-            // lane at a time so that their words are in flight together
+        for (int m = 0; m < CPT; ++m)
+            xv[m] = fma(alpha, pn[m], xv[m]);
+        if (G > 1) {
+            // the neighbours' boundary rows, a few cells a lane at a time so
+            // that their words are in flight together
             constexpr int NB = 4;
-            constexpr int NH = NT - kWave;
-            for (int e1 = t - kWave; e1 < 2 * n0; e1 += NB * NH) {
+            for (int e1 = t; e1 < 2 * n0; e1 += NB * NT) {
                 Word w[NB][2];
                 unsigned polls = 0;
                 for (;;) {
                     bool all = true;
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
-                        const int e = e1 + b * NH;
+                        const int e = e1 + b * NT;
                         const int side = e >= n0 ? 1 : 0, i = e - side * n0;
                         const bool want = e < 2 * n0 && (side == 0 ? has_top : has_bot);
                         // the top halo row is the bottom row of the strip above
@@ -520,45 +642,44 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop(Geo g, CoopGrid cg, doubl
                     if (all)
                         break;
                     if (++polls >= kCoopSpin) {
-                        sh_stall = 1;
+                        sh.stall = 1;
                         break;
                     }
                 }
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    if (e1 + b * NH < 2 * n0)
-                        hr[e1 + b * NH] = value_of(w[b][0], w[b][1]);
+                for (int b = 0; b < NB; ++b) {
+                    const int e = e1 + b * NT;
+                    if (e < 2 * n0)
+                        hz[e] = hd[e] * value_of(w[b][0], w[b][1]);
+                }
             }
         }
-        __syncthreads();
-        if (sh_stall || sh_stop)
+        __syncthreads(); // E
+        if (sh.stall || its >= max_its)
             break;
-        beta = sh_ab[1];
+        beta = sh.beta;
         first = false;
     }
     // x, r and the direction back to memory (a later launch resumes from
-    // them), and the state from workgroup 0
-    if (sh_stall)
-        fs.stalled = 1;
-    if (gid == 0 && t == 0)
-        *st = fs;
+    // them; after a stop the direction is one ahead and nobody's)
 #pragma unroll
     for (int m = 0; m < CPT; ++m)
-        if (sl.own >> m & 1) {
+        if (own[m]) {
             const int64_t c = padded(wi[m]);
             x[c] = xv[m];
             r[c] = rv[m];
-            pg[c] = pw[wi[m]];
+            pg[c] = pn[m];
         }
 }
 
 template <int NT, int CPT>
 const void* coop_kernel(int G)
 {
-    static_assert(kCoopMaxGroups <= 4 * kWave, "gather bucket");
-    return G <= kWave       ? (const void*)k_pcg_solve_coop<NT, CPT, 1>
-           : G <= 2 * kWave ? (const void*)k_pcg_solve_coop<NT, CPT, 2>
-                            : (const void*)k_pcg_solve_coop<NT, CPT, 4>;
+    static_assert(kCoopMaxGroups <= 8 * 32, "gather bucket");
+    return G <= 32    ? (const void*)k_pcg_solve_coop<NT, CPT, 1>
+           : G <= 64  ? (const void*)k_pcg_solve_coop<NT, CPT, 2>
+           : G <= 128 ? (const void*)k_pcg_solve_coop<NT, CPT, 4>
+                      : (const void*)k_pcg_solve_coop<NT, CPT, 8>;
 }
 
 // ---- 3-D grids ------------------------------------------------------------------------
@@ -586,22 +707,22 @@ __device__ __forceinline__ unsigned fresh(unsigned v)
     return v;
 }
 
-template <int NT, int CPT, int PPL>
-__global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
-                                                        double* __restrict__ x,
-                                                        double* __restrict__ r,
-                                                        double* __restrict__ pg, PcgState* st,
-                                                        CoopXch xc, int max_its)
+template <int NT, int CPT, int PQ>
+__global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
+                                                                double* __restrict__ x,
+                                                                double* __restrict__ r,
+                                                                double* __restrict__ pg,
+                                                                PcgState* st, CoopXch xc,
+                                                                int max_its)
 {
     if (blockIdx.x % cg.every)
         return;
+    constexpr int NW = NT / kWave;
     extern __shared__ double lds[];
     double* pw = lds;            // the direction window
     double* tab = lds + cg.nwin; // diag[0..6], then dinv[0..6]
     double* xl = tab + 14;       // x of the lane's cells, CPT per lane
-    __shared__ double red[2][2][NT / kWave];
-    __shared__ double sh_ab[2]; // alpha, beta
-    __shared__ int sh_stop, sh_stall;
+    __shared__ CoopShared<NW> sh;
     PcgState fs = *st; // read once, as in k_pcg_solve_coop
     const int t = threadIdx.x;
     const int gid = blockIdx.x / cg.every, G = cg.G;
@@ -610,9 +731,8 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
     const int nby = min(cg.by, n1 - j0), nbz = min(cg.bz, n2 - k0);
     const double s = offdiag<double>(g);
     const double ring0 = copysign(0.0, s);
-    if (t == 0)
-        sh_stall = 0;
-    for (int e = t; e < cg.nwin; e += NT)
+    sh.clear(t);
+    for (int e = t; e < cg.nwin; e += NT + kWave)
         pw[e] = ring0;
 #pragma unroll
     for (int q = 0; q < 7; ++q)
@@ -623,6 +743,16 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
     __syncthreads();
     if (fs.done)
         return;
+    if (__builtin_amdgcn_readfirstlane(t / kWave) == NW) {
+        __syncthreads(); // the cells are loaded
+        coop_scalars<NW, PQ>(sh, fs, gid, G, xc, g.periodic[0], max_its);
+        if (gid == 0 && t == NT) {
+            if (sh.stall)
+                fs.stalled = 1;
+            *st = fs;
+        }
+        return;
+    }
     bool first = fs.iter == 0;
     double beta = fs.beta;
     auto cell_cnt = [&](int i, int j, int k) -> int {
@@ -635,18 +765,17 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
     // halo cells: the rows y-low, y-high (nbz each), z-low, z-high (nby each).
     // hw: window index (bits 0-15), SOLID wall count (bits 16-18), kept only
     // where the row exists; hs: the cell's number.
-    constexpr int NH = NT - kWave;
     const int nrow = 2 * (nby + nbz);
     int hw[kCoopHalo], hs[kCoopHalo];
-    double hr[kCoopHalo];
+    double hz[kCoopHalo]; // D^-1 r
     unsigned halo_bits = 0;
 #pragma unroll
     for (int b = 0; b < kCoopHalo; ++b) {
         hw[b] = hs[b] = 0;
-        hr[b] = 0.0;
-        const int h = t - kWave + NH * b;
+        hz[b] = 0.0;
+        const int h = t + NT * b;
         const int row = h / n0, i = h - row * n0;
-        if (t < kWave || row >= nrow)
+        if (row >= nrow)
             continue;
         int jj, kk; // pencil-relative
         if (row < 2 * nbz) {
@@ -673,21 +802,21 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
         hw[b] = w | cell_cnt(i, j, k) << 16;
         hs[b] = i + n0 * (j + n1 * k);
         const int64_t c = padded(i, j, k);
-        hr[b] = r[c];
+        hz[b] = tab[7 + (hw[b] >> 16)] * r[c];
         if (!first)
             pw[w] = pg[c];
     }
 
     // own cells: window index, and SOLID wall count (bits 16-18)
     int wi[CPT], no[CPT]; // no: the cell's number
-    double rv[CPT], qv[CPT];
+    double rv[CPT], qv[CPT], pn[CPT];
     unsigned own_bits = 0, edge_bits = 0; // edge: some pencil's halo
     const int ncell = n0 * nby * nbz;
 #pragma unroll
     for (int m = 0; m < CPT; ++m) {
         wi[m] = 1 + e0 + e1; // pencil cell (0, 0, 0)
         no[m] = 0;
-        rv[m] = qv[m] = 0.0;
+        rv[m] = qv[m] = pn[m] = 0.0;
         const int L = t + NT * m;
         if (L < ncell) {
             const int row = L / n0, i = L - row * n0;
@@ -701,7 +830,7 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
             rv[m] = r[c];
             xl[L] = x[c];
             if (!first)
-                pw[wi[m] & 0xffff] = pg[c];
+                pn[m] = pg[c];
         }
     }
     __syncthreads();
@@ -709,10 +838,6 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
     for (int its = 1;; ++its) {
         const unsigned own = fresh(own_bits), edge = fresh(edge_bits), have = fresh(halo_bits);
         // direction: p = D^-1 r, or fma(beta, p, D^-1 r), own and halo cells
-        double pn[CPT];
-#pragma unroll
-        for (int m = 0; m < CPT; ++m)
-            pn[m] = pw[wi[m] & 0xffff];
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const double z = tab[7 + (wi[m] >> 16)] * rv[m];
@@ -725,11 +850,10 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
 #pragma unroll
         for (int b = 0; b < kCoopHalo; ++b)
             if (have >> b & 1) {
-                const double z = tab[7 + (hw[b] >> 16)] * hr[b];
                 double* pp = pw + (hw[b] & 0xffff);
-                *pp = first ? z : fma(beta, *pp, z);
+                *pp = first ? hz[b] : fma(beta, *pp, hz[b]);
             }
-        __syncthreads();
+        __syncthreads(); // A
         if (g.periodic[0]) {
             for (int q = t; q < nby * nbz; q += NT) {
                 double* row = pw + e0 * (q % nby + 1) + e1 * (q / nby + 1);
@@ -739,7 +863,7 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
             __syncthreads();
         }
         // q = A p in the stencil order {0}, -x, +x, -y, +y, -z, +z; p.q
-        double h1[1] = {0.0}, l1[1] = {0.0};
+        double h1 = 0.0, l1 = 0.0;
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
             const double* pp = pw + (wi[m] & 0xffff);
@@ -752,20 +876,17 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
             y = fma(s, pp[-e1], y);
             y = fma(s, pp[e1], y);
             qv[m] = mine ? y : 0.0;
-            dd_acc_prod(h1[0], l1[0], mine ? pn[m] : 0.0, qv[m]);
+            dd_acc_prod(h1, l1, mine ? pn[m] : 0.0, qv[m]);
         }
-        {
-            double pq[1];
-            coop_reduce<NT, 1, PPL>(h1, l1, gid, G, xc.part, 0, ++seq, red, &sh_stall, pq, [] {});
-            if (t == 0) {
-                fs.alpha = fs.rho / pq[0];
-                sh_ab[0] = fs.alpha;
-            }
-        }
-        __syncthreads();
-        if (sh_stall)
+        leave_pq(sh, h1, l1);
+        __syncthreads(); // B
+        if (sh.stop)
             break;
-        const double alpha = sh_ab[0];
+        ++seq;
+        __syncthreads(); // C
+        if (sh.stall)
+            break;
+        const double alpha = sh.alpha;
         // r = fma(-alpha, q, r), published where a neighbour needs it; r.r and
         // r.(D^-1 r); x = fma(alpha, p, x)
         double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
@@ -785,21 +906,12 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
             dd_acc_prod(hi[0], lo[0], rv[m], rv[m]);
             dd_acc_prod(hi[1], lo[1], rv[m], z);
         }
-        {
-            double rr[2];
-            coop_reduce<NT, 2, PPL>(hi, lo, gid, G, xc.part, 8, seq, red, &sh_stall, rr, [&] {
+        leave_rr(sh, hi, lo);
+        __syncthreads(); // D
 #pragma unroll
-                for (int m = 0; m < CPT; ++m)
-                    xl[t + NT * m] = fma(alpha, pw[wi[m] & 0xffff], xl[t + NT * m]);
-            });
-            if (t == 0) {
-                finish_update(&fs, rr[0], rr[1]);
-                sh_stop = fs.done || its >= max_its;
-                sh_ab[1] = fs.beta;
-            }
-        }
-        // the halo cells' new r (none in the gathering wave), four a lane at a
-        // time
+        for (int m = 0; m < CPT; ++m)
+            xl[t + NT * m] = fma(alpha, pn[m], xl[t + NT * m]);
+        // the halo cells' new r, four a lane at a time
 #pragma unroll
         for (int b0 = 0; b0 < kCoopHalo; b0 += 4) {
             if (!(have >> b0 & 15))
@@ -822,24 +934,20 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
                 if (all)
                     break;
                 if (++polls >= kCoopSpin) {
-                    sh_stall = 1;
+                    sh.stall = 1;
                     break;
                 }
             }
 #pragma unroll
             for (int b = 0; b < 4; ++b)
-                hr[b0 + b] = value_of(w[b][0], w[b][1]);
+                hz[b0 + b] = tab[7 + (hw[b0 + b] >> 16)] * value_of(w[b][0], w[b][1]);
         }
-        __syncthreads();
-        if (sh_stall || sh_stop)
+        __syncthreads(); // E
+        if (sh.stall || its >= max_its)
             break;
-        beta = sh_ab[1];
+        beta = sh.beta;
         first = false;
     }
-    if (sh_stall)
-        fs.stalled = 1;
-    if (gid == 0 && t == 0)
-        *st = fs;
 #pragma unroll
     for (int m = 0; m < CPT; ++m)
         if (own_bits >> m & 1) {
@@ -847,7 +955,7 @@ __global__ __launch_bounds__(NT) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
             const int64_t c = padded(i, row % n1, row / n1);
             x[c] = xl[t + NT * m];
             r[c] = rv[m];
-            pg[c] = pw[wi[m] & 0xffff];
+            pg[c] = pn[m];
         }
 }
 
@@ -861,11 +969,11 @@ size_t coop3_lds(const Coop3Grid& c)
 // in us, from measured parts: an exchange of G workgroups (twice), a cell of
 // a lane per wave of a SIMD, the fixed chain, and the halo words' traffic.
 // G = 0: none fits (more than 256 pencils of 4096 cells, about 100^3).  us per
-// iteration, the streaming tiles before and this: 45 x 52 x 61 22.6 -> 8.9,
-// 64^3 22.9 -> 9.6, 96^3 30.6 -> 15.3, 100^3 32 -> 17.6.
+// iteration, the streaming tiles and this: 45 x 52 x 61 22.6, 7.5; 64^3 22.9,
+// 8.2; 96^3 30.6, 13.7; 100^3 32, 15.8.
 Coop3Grid coop3_grid(const Geo& g)
 {
-    constexpr int shape[][2] = {{256, 2}, {256, 4}, {512, 4}, {512, 8}};
+    constexpr int shape[][2] = {{256, 2}, {256, 4}, {512, 4}, {448, 10}};
     Coop3Grid best{};
     double cost = 1e30;
     const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
@@ -875,7 +983,7 @@ Coop3Grid coop3_grid(const Geo& g)
         for (int bz = 1; bz <= n2 && bz <= 64; ++bz) {
             const int64_t cells = (int64_t)n0 * by * bz;
             const int64_t G64 = (int64_t)((n1 + by - 1) / by) * ((n2 + bz - 1) / bz);
-            if (cells > 4096 || G64 > kCoopMaxGroups)
+            if (cells > kCoopCells || G64 > kCoopMaxGroups)
                 continue;
             const int G = (int)G64;
             int q = 0;
@@ -893,11 +1001,11 @@ Coop3Grid coop3_grid(const Geo& g)
             c.nwin = c.e1 * (bz + 2);
             c.nt = nt;
             c.cpt = cpt;
-            if (halo > kCoopHalo * (nt - kWave) || c.nwin >= 1 << 16 ||
+            if (halo > kCoopHalo * nt || c.nwin >= 1 << 16 ||
                 coop3_lds(c) > 150 * 1024)
                 continue;
             const double us = 2.0 * (1.3 + 0.1 * std::log2((double)G) + 0.006 * G) + 1.5 +
-                              0.25 * (nt / 256) * cpt + 1e-3 * halo / (nt - kWave) * 200.0 +
+                              0.25 * (nt * cpt) / 256.0 + 1e-3 * halo / nt * 200.0 +
                               3.2e-6 * halo * G;
             if (us < cost) {
                 cost = us;
@@ -914,9 +1022,10 @@ Coop3Grid coop3_grid(const Geo& g)
 template <int NT, int CPT>
 const void* coop3_kernel(int G)
 {
-    return G <= kWave       ? (const void*)k_pcg_solve_coop3<NT, CPT, 1>
-           : G <= 2 * kWave ? (const void*)k_pcg_solve_coop3<NT, CPT, 2>
-                            : (const void*)k_pcg_solve_coop3<NT, CPT, 4>;
+    return G <= 32    ? (const void*)k_pcg_solve_coop3<NT, CPT, 1>
+           : G <= 64  ? (const void*)k_pcg_solve_coop3<NT, CPT, 2>
+           : G <= 128 ? (const void*)k_pcg_solve_coop3<NT, CPT, 4>
+                      : (const void*)k_pcg_solve_coop3<NT, CPT, 8>;
 }
 
 } // namespace
@@ -973,18 +1082,18 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
         xc.halo = xc.part + (size_t)c3.G * 16;
         fn = c3.nt == 256 ? (c3.cpt == 2 ? coop3_kernel<256, 2>(c3.G) : coop3_kernel<256, 4>(c3.G))
              : c3.cpt == 4 ? coop3_kernel<512, 4>(c3.G)
-                           : coop3_kernel<512, 8>(c3.G);
+                           : coop3_kernel<448, 10>(c3.G);
         grid = dim3(c3.G * c3.every);
-        block = dim3(c3.nt);
+        block = dim3(c3.nt + kWave);
         lds = coop3_lds(c3);
     } else {
         cg = coop_grid(g);
         xc.halo = xc.part + (size_t)cg.G * 16;
         fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
              : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
-                           : coop_kernel<512, 8>(cg.G);
+                           : coop_kernel<448, 10>(cg.G);
         grid = dim3(cg.G * cg.every);
-        block = dim3(cg.nt);
+        block = dim3(cg.nt + kWave);
         lds = coop_lds(g, cg);
     }
     const hipError_t e = hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
