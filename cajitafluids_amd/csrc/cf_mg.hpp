@@ -119,6 +119,7 @@ struct MgFused
 {
     int dim, n[3], periodic[3];
     int tiles_x, core_x, tiles_y, core_y, nchunk, kz, work;
+    int waves; // of a block
     double alpha;
     double coupling; // of every pair of neighbours, or 0 if they differ
     MgParentMap lv, pm;

@@ -34,7 +34,6 @@
 // copied at the loop's end (settle()).
 #include <hip/hip_runtime.h>
 
-#include <climits>
 #include <type_traits>
 
 #include "cf_mg.hpp"
@@ -52,13 +51,15 @@ namespace
 // up in FP64: 121 and 313 us against 113 and 121).
 constexpr int RY = 2;
 
-// Waves per block, all resident at once: as many as the registers of a leg
+// Waves per block of the large levels, all resident at once: as many as the registers of a leg
 // allow (FP32 16 against 12: 29 and 39 against 34 and 43 us, 190 x 182 x 149).
 template <class T, bool UNI>
 constexpr int waves_of()
 {
     return std::is_same<T, float>::value || UNI ? 16 : 12;
 }
+// Waves per block of the 3-D levels that fill the GPU no other way (tile_level).
+constexpr int kSmallLeg = 8;
 // Steps from a plane's loads to their use.
 template <class T, bool UNI>
 constexpr int ahead_of()
@@ -711,27 +712,38 @@ void split_axis(int n, bool periodic, int ext, int below, int above, int& tiles,
         core = mid;
 }
 
-// The tiling of a level: the planes of a chunk (even, so that a block has
-// both children of a parent along z) that minimise the last CU's blocks
-// times a block's steps.
-void tile_level(MgFused& f, int nu, int waves)
+// The tiling of a level: the waves of a block (`big`, or in 3-D kSmallLeg) and
+// the planes of a chunk (even, so that a block has both children of a parent
+// along z) that minimise the last CU's blocks times a block's steps times a
+// step's time, which 8 waves take in 0.65 of 16's or 12's (1.2-1.35 us).  Half
+// the rows a block cost a large level a third more overlap; a level that
+// leaves CUs idle gets shorter steps.  us a leg, 16 or 12 waves and 8: 128^3
+// 25.0, 29.1; 64^3 16.9, 12.2; 32^3 16.4, 11.6; 95 x 91 x 75 (boxes) 19.0,
+// 16.8; 47 x 45 x 37 15.7, 13.0.
+void tile_level(MgFused& f, int nu, int big)
 {
-    int64_t best = INT64_MAX;
-    MgFused t = f;
-    split_axis(t.n[0], t.periodic[0], kWave, nu, nu, t.tiles_x, t.core_x);
-    split_axis(t.n[1], t.periodic[1], RY * waves, (nu + 1) / 2 * 2, nu, t.tiles_y, t.core_y);
-    const int tiles = t.tiles_x * t.tiles_y;
-    for (int kz = 2;; kz += 2) {
-        t.kz = t.dim == 3 ? kz : 1;
-        t.nchunk = (t.n[2] + t.kz - 1) / t.kz;
-        t.work = tiles * t.nchunk;
-        const int64_t cost = (int64_t)((t.work + 255) / 256) * (t.kz + 2 * nu);
-        if (cost < best && t.work <= kRedBlocks) {
-            best = cost;
-            f = t;
-        }
-        if (t.dim == 2 || kz >= t.n[2])
+    double best = 1e30;
+    for (int waves : {big, kSmallLeg}) {
+        if (waves != big && f.dim == 2)
             break;
+        MgFused t = f;
+        t.waves = waves;
+        split_axis(t.n[0], t.periodic[0], kWave, nu, nu, t.tiles_x, t.core_x);
+        split_axis(t.n[1], t.periodic[1], RY * waves, (nu + 1) / 2 * 2, nu, t.tiles_y, t.core_y);
+        const int tiles = t.tiles_x * t.tiles_y;
+        for (int kz = 2;; kz += 2) {
+            t.kz = t.dim == 3 ? kz : 1;
+            t.nchunk = (t.n[2] + t.kz - 1) / t.kz;
+            t.work = tiles * t.nchunk;
+            const double cost = (double)((t.work + 255) / 256) * (t.kz + 2 * nu) *
+                                (waves == big ? 1.0 : 0.65);
+            if (cost < best && t.work <= kRedBlocks) {
+                best = cost;
+                f = t;
+            }
+            if (t.dim == 2 || kz >= t.n[2])
+                break;
+        }
     }
 }
 
@@ -765,9 +777,13 @@ template <class T, class TB, class TP, int NU, bool UP, bool RZ, bool UNI>
 void leg3(const MgFused& f, const MgOpTab<T>* tab, const TB* b, const T* x, const TP* xc, T* xo,
           TP* bc, PcgState* st, RedBuf rb, hipStream_t s)
 {
-    constexpr int NW = waves_of<T, UNI>();
-    hipLaunchKernelGGL((k_mg_leg3<T, TB, TP, NU, UP, RZ, UNI, NW>), dim3((f.work + 7) / 8 * 8),
-                       dim3(NW * kWave), 0, s, f, tab, b, x, xc, xo, bc, st, rb);
+    const dim3 grid((f.work + 7) / 8 * 8), block(f.waves * kWave);
+    if (f.waves == kSmallLeg)
+        hipLaunchKernelGGL((k_mg_leg3<T, TB, TP, NU, UP, RZ, UNI, kSmallLeg>), grid, block, 0, s,
+                           f, tab, b, x, xc, xo, bc, st, rb);
+    else
+        hipLaunchKernelGGL((k_mg_leg3<T, TB, TP, NU, UP, RZ, UNI, waves_of<T, UNI>()>), grid,
+                           block, 0, s, f, tab, b, x, xc, xo, bc, st, rb);
 }
 
 template <int NU, bool UP, bool RZ, bool UNI>

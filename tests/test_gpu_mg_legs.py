@@ -25,11 +25,23 @@ GRIDS = [
 @pytest.mark.parametrize("nu", [2, 3, 4])
 @pytest.mark.parametrize("n,periodic", GRIDS)
 def test_mg_legs(oracle_mod, n, periodic, nu, precision):
-    from cajitafluids_amd import _lib
-    from cajitafluids_amd.solver import Solver
     dim = 3 if n[2] > 1 else 2
     if dim == 2 and precision != K.FP64:
         pytest.skip("FP32 levels are 3-D")
+    check_solve(oracle_mod, n, periodic, nu, precision)
+
+
+# levels whose legs run in blocks of 16 and of 12 waves: level 0, and levels 0
+# (padded) and 1 (boxes)
+@pytest.mark.parametrize("n,periodic", [((130, 121, 96), (0, 1, 0)), ((247, 243, 159), (0, 0, 0))])
+def test_mg_legs_large(oracle_mod, n, periodic):
+    check_solve(oracle_mod, n, periodic, 3, K.FP64)
+
+
+def check_solve(oracle_mod, n, periodic, nu, precision):
+    from cajitafluids_amd import _lib
+    from cajitafluids_amd.solver import Solver
+    dim = 3 if n[2] > 1 else 2
     cfg = K.base_config(dim, n[0])
     cfg.update(num_cell=list(n), hi=[1.0, n[1] / n[0], n[2] / n[0] if dim == 3 else 1.0],
                clamp_dt=0, dt=0.002, halo=1, field_order=1, periodic=list(periodic),
