@@ -19,7 +19,7 @@ void hip_check(hipError_t e, const char* what)
 }
 
 template <class T>
-void DevArray<T>::alloc(int64_t count, hipStream_t s)
+void DevArray<T>::alloc(int64_t count, hipStream_t s, bool zero)
 {
     release();
     void* p = nullptr;
@@ -32,7 +32,8 @@ void DevArray<T>::alloc(int64_t count, hipStream_t s)
     }
     ptr = (T*)p;
     n = count;
-    CF_HIP(hipMemsetAsync(ptr, 0, (size_t)count * sizeof(T), s));
+    if (zero)
+        CF_HIP(hipMemsetAsync(ptr, 0, (size_t)count * sizeof(T), s));
 }
 
 template struct DevArray<double>;

@@ -56,7 +56,7 @@ struct DevArray
     DevArray(const DevArray&) = delete;
     DevArray& operator=(const DevArray&) = delete;
     ~DevArray() { release(); }
-    void alloc(int64_t count, hipStream_t s);
+    void alloc(int64_t count, hipStream_t s, bool zero = true);
     void release()
     {
         if (ptr)
