@@ -66,6 +66,18 @@ __device__ __forceinline__ void dd_norm(double& hi, double& lo)
     hi = s;
 }
 
+// (hi, lo) += (oh, ol): the high parts' rounding error goes to the low part,
+// which is summed as it is (as in dd_acc_prod): one addition a step is on the
+// high parts' chain instead of dd_add's seven.
+__device__ __forceinline__ void dd_merge(double& hi, double& lo, double oh, double ol)
+{
+    const double s = hi + oh;
+    const double t = s - hi;
+    const double e = (hi - (s - t)) + (oh - t);
+    lo = (lo + ol) + e;
+    hi = s;
+}
+
 // ---- B-spline sampling (Cajita SplineData / evaluateSpline / G2P::value,
 // called at src/Interpolation.hpp:30-41) -------------------------------------
 // Weights at the fraction t of a logical coordinate.

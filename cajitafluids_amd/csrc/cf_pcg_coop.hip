@@ -140,65 +140,12 @@ __device__ __forceinline__ double value_of(Word lo, Word hi)
     return __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffu)));
 }
 
-// A lane's value from lane ^ 1, ^ 2, and (where lanes of a quad, then of
-// eight, hold the same) from the other quad of eight and the other eight of
-// sixteen; from lane ^ 16 and ^ 32.
-template <int CTRL>
-__device__ __forceinline__ double move_row(double v)
-{
-    return __hiloint2double(
-        __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
-        __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
-}
-template <int W>
-__device__ __forceinline__ double move_half(double v)
-{
-    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
-    const bool up = (threadIdx.x & W) != 0;
-    if constexpr (W == 16) {
-        const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-        const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
-    } else {
-        const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-        const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
-    }
-}
-
-// (hi, lo) += (oh, ol): the high parts' rounding error goes to the low part,
-// which is summed as it is (as in dd_acc_prod): one addition a step is on the
-// high parts' chain instead of dd_add's seven.
-__device__ __forceinline__ void dd_merge(double& hi, double& lo, double oh, double ol)
-{
-    const double s = hi + oh;
-    const double t = s - hi;
-    const double e = (hi - (s - t)) + (oh - t);
-    lo = (lo + ol) + e;
-    hi = s;
-}
 #define CF_STEP(MOVE)                                   \
     {                                                   \
         const double oh = MOVE(h), ol = MOVE(l);        \
         dd_merge(h, l, oh, ol);                         \
     }
 
-// Sum of (h, l) over groups of `width` lanes (a power of two), in each of them.
-__device__ __forceinline__ void wave_sum(double& h, double& l, int width)
-{
-    if (width > 1)
-        CF_STEP(move_row<0xB1>) // quad_perm 1 0 3 2
-    if (width > 2)
-        CF_STEP(move_row<0x4E>) // quad_perm 2 3 0 1
-    if (width > 4)
-        CF_STEP(move_row<0x141>) // row_half_mirror
-    if (width > 8)
-        CF_STEP(move_row<0x140>) // row_mirror
-    if (width > 16)
-        CF_STEP(move_half<16>)
-    if (width > 32)
-        CF_STEP(move_half<32>)
-}
 // The sums over the even lanes and over the odd lanes, in each even and each
 // odd lane, of values that repeat every `width` lanes or (width >= 16) are
 // zero past them.  As in wave_sum, the two lanes of a step add the same two

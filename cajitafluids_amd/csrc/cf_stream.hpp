@@ -24,46 +24,97 @@
 namespace cfmi
 {
 
-// ---- grid reduction ----------------------------------------------------------
-// Each block reduces its lanes' double-double sums (xor shuffles, then LDS),
-// and thread 0 publishes the block's partial with agent-scope atomic stores
-// (written through to memory, so every XCD sees them), waits for them to
-// complete, and counts its arrival with agent-scope atomics (per group of
-// blocks, then per group).  The block that arrives last reads all partials
-// with agent-scope atomic loads (which
-// read memory, not its own XCD's L2), reduces them and runs `fin` on thread
-// 0.  No fence is issued: an agent-scope fence would write back and
-// invalidate the XCD's whole L2 on every block.
-template <int NV, int BS = kBlock>
-__device__ __forceinline__ void block_reduce(double (&hi)[NV], double (&lo)[NV])
+// ---- wave sums -------------------------------------------------------------------
+// A lane's value from lane ^ 1, ^ 2, and (where lanes of a quad, then of
+// eight, hold the same) from the other quad of eight and the other eight of
+// sixteen; from lane ^ 16 and ^ 32.
+template <int CTRL>
+__device__ __forceinline__ double move_row(double v)
 {
-    __shared__ double sh[NV][2][BS / kWave];
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            double oh = __shfl_xor(hi[v], off, kWave);
-            double ol = __shfl_xor(lo[v], off, kWave);
-            dd_add(hi[v], lo[v], oh, ol);
-        }
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true));
+}
+template <int W>
+__device__ __forceinline__ double move_half(double v)
+{
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    const bool up = (threadIdx.x & W) != 0;
+    if constexpr (W == 16) {
+        const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
+    } else {
+        const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double((int)(up ? b[0] : b[1]), (int)(up ? a[0] : a[1]));
     }
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wv = threadIdx.x / kWave;
-    if (lane == 0) {
+}
+
+#define CF_STEP(MOVE)                                   \
+    {                                                   \
+        const double oh = MOVE(h), ol = MOVE(l);        \
+        dd_merge(h, l, oh, ol);                         \
+    }
+
+// Sum of (h, l) over groups of `width` lanes (a power of two), in each of them.
+__device__ __forceinline__ void wave_sum(double& h, double& l, int width)
+{
+    if (width > 1)
+        CF_STEP(move_row<0xB1>) // quad_perm 1 0 3 2
+    if (width > 2)
+        CF_STEP(move_row<0x4E>) // quad_perm 2 3 0 1
+    if (width > 4)
+        CF_STEP(move_row<0x141>) // row_half_mirror
+    if (width > 8)
+        CF_STEP(move_row<0x140>) // row_mirror
+    if (width > 16)
+        CF_STEP(move_half<16>)
+    if (width > 32)
+        CF_STEP(move_half<32>)
+}
+#undef CF_STEP
+
+// ---- grid reduction ----------------------------------------------------------
+// Each block sums its lanes' double-double values, thread 0 publishes the
+// block's partial with agent-scope atomic stores (written through to memory,
+// so every XCD sees them), waits for them to complete, and counts its arrival
+// with agent-scope atomics (per group of blocks, then per group).  The block
+// that arrives last reads all partials with agent-scope atomic loads (which
+// read memory, not its own XCD's L2), sums them and runs `fin` on thread 0.
+// No fence is issued: an agent-scope fence would write back and invalidate
+// the XCD's whole L2 on every block.
+//
+// A block's sum: lane moves and dd_merge, the waves' sums in one wave's lanes.
+// With LDS permutes, dd_add and the waves one after the other it was 1.5 us of
+// a 2-D PCG kernel's 9.4-10.6 (391 x 263) and of an upward multigrid leg's 9.1.
+// Numbered words that block 0 polls, instead of the counted arrivals, cost
+// the large grids their bandwidth while it polls: 256^3 190 -> 214 us an
+// iteration (203 with a pause between polls), and gained nothing on small ones.
+
+// The block's sums, in every lane of its first wave.
+template <int NV, int BS = kBlock>
+__device__ __forceinline__ void block_sum(double (&hi)[NV], double (&lo)[NV])
+{
+    constexpr int NW = BS / kWave, N = NW <= 4 ? 4 : NW <= 8 ? 8 : 16;
+    __shared__ double sh[NV][2][N];
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
+    for (int v = 0; v < NV; ++v) {
+        wave_sum(hi[v], lo[v], kWave);
+        if (lane == 0) {
             sh[v][0][wv] = hi[v];
             sh[v][1][wv] = lo[v];
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (wv == 0) {
+        const int w = lane & (N - 1);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            hi[v] = sh[v][0][0];
-            lo[v] = sh[v][1][0];
-            for (int w = 1; w < BS / kWave; ++w)
-                dd_add(hi[v], lo[v], sh[v][0][w], sh[v][1][w]);
+            hi[v] = NW == N || w < NW ? sh[v][0][w] : 0.0;
+            lo[v] = NW == N || w < NW ? sh[v][1][w] : 0.0;
+            wave_sum(hi[v], lo[v], N);
         }
     }
     __syncthreads();
@@ -73,7 +124,7 @@ template <int NV, int BS = kBlock, class Fin>
 __device__ __forceinline__ void grid_reduce(double (&hi)[NV], double (&lo)[NV],
                                             RedBuf rb, Fin&& fin)
 {
-    block_reduce<NV, BS>(hi, lo);
+    block_sum<NV, BS>(hi, lo);
     __shared__ int last;
     if (threadIdx.x == 0) {
         double* part = rb.partials + (size_t)blockIdx.x * NV * 2;
@@ -116,11 +167,10 @@ __device__ __forceinline__ void grid_reduce(double (&hi)[NV], double (&lo)[NV],
     __syncthreads();
     if (!last)
         return;
-    double h2[NV], l2[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        h2[v] = 0.0;
-        l2[v] = 0.0;
+        hi[v] = 0.0;
+        lo[v] = 0.0;
     }
     for (int b = threadIdx.x; b < (int)gridDim.x; b += BS) {
         double* part = rb.partials + (size_t)b * NV * 2;
@@ -130,15 +180,15 @@ __device__ __forceinline__ void grid_reduce(double (&hi)[NV], double (&lo)[NV],
                                                 __HIP_MEMORY_SCOPE_AGENT);
             const double pl = __hip_atomic_load(
                 &part[2 * v + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            dd_add(h2[v], l2[v], ph, pl);
+            dd_add(hi[v], lo[v], ph, pl);
         }
     }
-    block_reduce<NV, BS>(h2, l2);
+    block_sum<NV, BS>(hi, lo);
     if (threadIdx.x == 0) {
         double sum[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-            sum[v] = h2[v] + l2[v];
+            sum[v] = hi[v] + lo[v];
         fin(sum);
     }
     if (threadIdx.x < kCounterSlots)
