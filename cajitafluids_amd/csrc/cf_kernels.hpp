@@ -123,7 +123,7 @@ inline bool pcg_pairs_x(const Geo& g)
 // partials buffer).
 int reduction_blocks_max(const Geo& g);
 
-// FP64 Jacobi-PCG iterations in one cooperative launch of one workgroup per
+// Jacobi-PCG iterations (FP64, or on 3-D grids FP32) in one cooperative launch of one workgroup per
 // strip of rows (2-D) or pencil of x-rows (3-D), until the state's stop test or `max_its`
 // iterations of this launch (x, r and the direction p are read at the start
 // and written back at the end, so launches chain).  The same x, r, direction
@@ -136,8 +136,9 @@ int reduction_blocks_max(const Geo& g);
 // resident, or the device has no cooperative launch); nothing ran then.
 bool pcg_coop_fits(const Geo& g);
 size_t coop_xch_bytes(const Geo& g);
-bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgState* st,
-                           void* xch, unsigned& seq, int max_its, hipStream_t s);
+template <class T>
+bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* xch,
+                           unsigned& seq, int max_its, hipStream_t s);
 
 // FP32-inner / FP64-outer defect correction.  The host runs the outer loop
 // from the device-computed norms (one read-back per pass).

@@ -1,5 +1,6 @@
 // cf_pcg_coop.hip -- a whole FP64 PCG solve of a 2-D grid, or of a 3-D grid of
-// up to about 100^3 cells, in one cooperative launch.
+// up to about 100^3 cells, in one cooperative launch; on those 3-D grids also
+// the FP32 iterations of a pass of a refined solve.
 //
 // A 2-D streaming iteration at 128^2-512^2 is two launches whose time goes
 // to start-up, one sweep per lane group and the grid reduction's arrival
@@ -654,21 +655,56 @@ __device__ __forceinline__ unsigned fresh(unsigned v)
     return v;
 }
 
-template <int NT, int CPT, int PQ>
+// The words of a value at place `at`: two of a double, one of a float.
+__device__ __forceinline__ void put_value(Word* base, int at, unsigned seq, double v)
+{
+    put_word(base + 2 * (size_t)at, seq, (unsigned)__double2loint(v));
+    put_word(base + 2 * (size_t)at + 1, seq, (unsigned)__double2hiint(v));
+}
+__device__ __forceinline__ void put_value(Word* base, int at, unsigned seq, float v)
+{
+    put_word(base + at, seq, __float_as_uint(v));
+}
+template <class T>
+struct ValueWords
+{
+    Word lo, hi;
+    __device__ __forceinline__ void get(const Word* base, int at)
+    {
+        lo = get_word(base + 2 * (size_t)at);
+        hi = get_word(base + 2 * (size_t)at + 1);
+    }
+    __device__ __forceinline__ bool is(unsigned seq) const
+    {
+        return (unsigned)(lo >> 32) == seq && (unsigned)(hi >> 32) == seq;
+    }
+    __device__ __forceinline__ T value() const { return value_of(lo, hi); }
+};
+template <>
+struct ValueWords<float>
+{
+    Word w;
+    __device__ __forceinline__ void get(const Word* base, int at) { w = get_word(base + at); }
+    __device__ __forceinline__ bool is(unsigned seq) const { return (unsigned)(w >> 32) == seq; }
+    __device__ __forceinline__ float value() const { return __uint_as_float((unsigned)w); }
+};
+
+template <class T, int NT, int CPT, int PQ>
 __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid cg,
-                                                                double* __restrict__ x,
-                                                                double* __restrict__ r,
-                                                                double* __restrict__ pg,
+                                                                T* __restrict__ x,
+                                                                T* __restrict__ r,
+                                                                T* __restrict__ pg,
                                                                 PcgState* st, CoopXch xc,
                                                                 int max_its)
 {
     if (blockIdx.x % cg.every)
         return;
     constexpr int NW = NT / kWave;
+    constexpr bool EXACT = std::is_same<T, float>::value; // products of two T in double
     extern __shared__ double lds[];
-    double* pw = lds;            // the direction window
-    double* tab = lds + cg.nwin; // diag[0..6], then dinv[0..6]
-    double* xl = tab + 14;       // x of the lane's cells, CPT per lane
+    T* pw = reinterpret_cast<T*>(lds); // the direction window
+    T* tab = pw + cg.nwin;             // diag[0..6], then dinv[0..6]
+    T* xl = tab + 14;                  // x of the lane's cells, CPT per lane
     __shared__ CoopShared<NW> sh;
     PcgState fs = *st; // read once, as in k_pcg_solve_coop
     const int t = threadIdx.x;
@@ -676,16 +712,16 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
     const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2], e0 = cg.e0, e1 = cg.e1;
     const int j0 = gid % cg.gy * cg.by, k0 = gid / cg.gy * cg.bz;
     const int nby = min(cg.by, n1 - j0), nbz = min(cg.bz, n2 - k0);
-    const double s = offdiag<double>(g);
-    const double ring0 = copysign(0.0, s);
+    const T s = offdiag<T>(g);
+    const T ring0 = s < (T)0 ? -(T)0 : (T)0; // a zero of s's sign
     sh.clear(t);
     for (int e = t; e < cg.nwin; e += NT + kWave)
         pw[e] = ring0;
 #pragma unroll
     for (int q = 0; q < 7; ++q)
         if (t == q) {
-            tab[q] = g.diag[q];
-            tab[7 + q] = g.dinv[q];
+            tab[q] = diag_of<T>(g, q);
+            tab[7 + q] = dinv_of<T>(g, q);
         }
     __syncthreads();
     if (fs.done)
@@ -701,7 +737,7 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
         return;
     }
     bool first = fs.iter == 0;
-    double beta = fs.beta;
+    T beta = (T)fs.beta;
     auto cell_cnt = [&](int i, int j, int k) -> int {
         return wall_count(g, 0, i) + wall_count(g, 1, j) + wall_count(g, 2, k);
     };
@@ -714,12 +750,12 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
     // where the row exists; hs: the cell's number.
     const int nrow = 2 * (nby + nbz);
     int hw[kCoopHalo], hs[kCoopHalo];
-    double hz[kCoopHalo]; // D^-1 r
+    T hz[kCoopHalo]; // D^-1 r
     unsigned halo_bits = 0;
 #pragma unroll
     for (int b = 0; b < kCoopHalo; ++b) {
         hw[b] = hs[b] = 0;
-        hz[b] = 0.0;
+        hz[b] = (T)0;
         const int h = t + NT * b;
         const int row = h / n0, i = h - row * n0;
         if (row >= nrow)
@@ -756,14 +792,15 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
 
     // own cells: window index, and SOLID wall count (bits 16-18)
     int wi[CPT], no[CPT]; // no: the cell's number
-    double rv[CPT], qv[CPT], pn[CPT];
+    T rv[CPT], qv[CPT], pn[CPT];
+    T po[CPT]; // FP32: the direction before, which the next pass resumes from
     unsigned own_bits = 0, edge_bits = 0; // edge: some pencil's halo
     const int ncell = n0 * nby * nbz;
 #pragma unroll
     for (int m = 0; m < CPT; ++m) {
         wi[m] = 1 + e0 + e1; // pencil cell (0, 0, 0)
         no[m] = 0;
-        rv[m] = qv[m] = pn[m] = 0.0;
+        rv[m] = qv[m] = pn[m] = po[m] = (T)0;
         const int L = t + NT * m;
         if (L < ncell) {
             const int row = L / n0, i = L - row * n0;
@@ -787,8 +824,10 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
         // direction: p = D^-1 r, or fma(beta, p, D^-1 r), own and halo cells
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
-            const double z = tab[7 + (wi[m] >> 16)] * rv[m];
-            pn[m] = first ? z : fma(beta, pn[m], z);
+            const T z = tab[7 + (wi[m] >> 16)] * rv[m];
+            if constexpr (EXACT)
+                po[m] = pn[m];
+            pn[m] = first ? z : fma_t<T>(beta, pn[m], z);
         }
 #pragma unroll
         for (int m = 0; m < CPT; ++m)
@@ -797,13 +836,13 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
 #pragma unroll
         for (int b = 0; b < kCoopHalo; ++b)
             if (have >> b & 1) {
-                double* pp = pw + (hw[b] & 0xffff);
-                *pp = first ? hz[b] : fma(beta, *pp, hz[b]);
+                T* pp = pw + (hw[b] & 0xffff);
+                *pp = first ? hz[b] : fma_t<T>(beta, *pp, hz[b]);
             }
         __syncthreads(); // A
         if (g.periodic[0]) {
             for (int q = t; q < nby * nbz; q += NT) {
-                double* row = pw + e0 * (q % nby + 1) + e1 * (q / nby + 1);
+                T* row = pw + e0 * (q % nby + 1) + e1 * (q / nby + 1);
                 row[0] = row[n0];
                 row[n0 + 1] = row[1];
             }
@@ -813,71 +852,70 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
         double h1 = 0.0, l1 = 0.0;
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
-            const double* pp = pw + (wi[m] & 0xffff);
+            const T* pp = pw + (wi[m] & 0xffff);
             const bool mine = own >> m & 1;
-            double y = tab[wi[m] >> 16] * pn[m];
-            y = fma(s, pp[-1], y);
-            y = fma(s, pp[1], y);
-            y = fma(s, pp[-e0], y);
-            y = fma(s, pp[e0], y);
-            y = fma(s, pp[-e1], y);
-            y = fma(s, pp[e1], y);
-            qv[m] = mine ? y : 0.0;
-            dd_acc_prod(h1, l1, mine ? pn[m] : 0.0, qv[m]);
+            T y = tab[wi[m] >> 16] * pn[m];
+            y = fma_t<T>(s, pp[-1], y);
+            y = fma_t<T>(s, pp[1], y);
+            y = fma_t<T>(s, pp[-e0], y);
+            y = fma_t<T>(s, pp[e0], y);
+            y = fma_t<T>(s, pp[-e1], y);
+            y = fma_t<T>(s, pp[e1], y);
+            qv[m] = mine ? y : (T)0;
+            dd_acc_prod<EXACT>(h1, l1, mine ? (double)pn[m] : 0.0, (double)qv[m]);
         }
         leave_pq(sh, h1, l1);
         __syncthreads(); // B
-        if (sh.stop)
+        if (sh.stop) {
+            if constexpr (EXACT) {
+#pragma unroll
+                for (int m = 0; m < CPT; ++m)
+                    pn[m] = po[m];
+            }
             break;
+        }
         ++seq;
         __syncthreads(); // C
         if (sh.stall)
             break;
-        const double alpha = sh.alpha;
+        const T alpha = (T)sh.alpha;
         // r = fma(-alpha, q, r), published where a neighbour needs it; r.r and
         // r.(D^-1 r); x = fma(alpha, p, x)
         double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
         ++seq;
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
-            rv[m] = fma(-alpha, qv[m], rv[m]);
+            rv[m] = fma_t<T>(-alpha, qv[m], rv[m]);
             if (edge >> m & 1) {
-                Word* hb = xc.halo + 2 * (size_t)no[m];
-                put_word(hb, seq, (unsigned)__double2loint(rv[m]));
-                put_word(hb + 1, seq, (unsigned)__double2hiint(rv[m]));
+                put_value(xc.halo, no[m], seq, rv[m]);
             }
         }
 #pragma unroll
         for (int m = 0; m < CPT; ++m) {
-            const double z = tab[7 + (wi[m] >> 16)] * rv[m];
-            dd_acc_prod(hi[0], lo[0], rv[m], rv[m]);
-            dd_acc_prod(hi[1], lo[1], rv[m], z);
+            const T z = tab[7 + (wi[m] >> 16)] * rv[m];
+            dd_acc_prod<EXACT>(hi[0], lo[0], (double)rv[m], (double)rv[m]);
+            dd_acc_prod<EXACT>(hi[1], lo[1], (double)rv[m], (double)z);
         }
         leave_rr(sh, hi, lo);
         __syncthreads(); // D
 #pragma unroll
         for (int m = 0; m < CPT; ++m)
-            xl[t + NT * m] = fma(alpha, pn[m], xl[t + NT * m]);
+            xl[t + NT * m] = fma_t<T>(alpha, pn[m], xl[t + NT * m]);
         // the halo cells' new r, four a lane at a time
 #pragma unroll
         for (int b0 = 0; b0 < kCoopHalo; b0 += 4) {
             if (!(have >> b0 & 15))
                 continue;
-            Word w[4][2];
+            ValueWords<T> w[4];
             unsigned polls = 0;
             for (;;) {
                 bool all = true;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const Word* hb = xc.halo + 2 * (size_t)hs[b0 + b];
-                    w[b][0] = get_word(hb);
-                    w[b][1] = get_word(hb + 1);
-                }
+                for (int b = 0; b < 4; ++b)
+                    w[b].get(xc.halo, hs[b0 + b]);
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
-                    all = all && (!(have >> (b0 + b) & 1) ||
-                                  ((unsigned)(w[b][0] >> 32) == seq &&
-                                   (unsigned)(w[b][1] >> 32) == seq));
+                    all = all && (!(have >> (b0 + b) & 1) || w[b].is(seq));
                 if (all)
                     break;
                 if (++polls >= kCoopSpin) {
@@ -887,12 +925,12 @@ __global__ __launch_bounds__(NT + kWave) void k_pcg_solve_coop3(Geo g, Coop3Grid
             }
 #pragma unroll
             for (int b = 0; b < 4; ++b)
-                hz[b0 + b] = tab[7 + (hw[b0 + b] >> 16)] * value_of(w[b][0], w[b][1]);
+                hz[b0 + b] = tab[7 + (hw[b0 + b] >> 16)] * w[b].value();
         }
         __syncthreads(); // E
         if (sh.stall || its >= max_its)
             break;
-        beta = sh.beta;
+        beta = (T)sh.beta;
         first = false;
     }
 #pragma unroll
@@ -917,7 +955,8 @@ size_t coop3_lds(const Coop3Grid& c)
 // a lane per wave of a SIMD, the fixed chain, and the halo words' traffic.
 // G = 0: none fits (more than 256 pencils of 4096 cells, about 100^3).  us per
 // iteration, the streaming tiles and this: 45 x 52 x 61 22.6, 7.5; 64^3 22.9,
-// 8.2; 96^3 30.6, 13.7; 100^3 32, 15.8.
+// 8.2; 96^3 30.6, 13.7; 100^3 32, 15.8.  FP32, a refined solve's time over its
+// iterations: 32^3 22, 6.7; 64^3 25, 7.8; 96^3 30, 12.6.
 Coop3Grid coop3_grid(const Geo& g)
 {
     constexpr int shape[][2] = {{256, 2}, {256, 4}, {512, 4}, {448, 10}};
@@ -966,13 +1005,20 @@ Coop3Grid coop3_grid(const Geo& g)
     return best;
 }
 
-template <int NT, int CPT>
+template <class T, int NT, int CPT>
 const void* coop3_kernel(int G)
 {
-    return G <= 32    ? (const void*)k_pcg_solve_coop3<NT, CPT, 1>
-           : G <= 64  ? (const void*)k_pcg_solve_coop3<NT, CPT, 2>
-           : G <= 128 ? (const void*)k_pcg_solve_coop3<NT, CPT, 4>
-                      : (const void*)k_pcg_solve_coop3<NT, CPT, 8>;
+    return G <= 32    ? (const void*)k_pcg_solve_coop3<T, NT, CPT, 1>
+           : G <= 64  ? (const void*)k_pcg_solve_coop3<T, NT, CPT, 2>
+           : G <= 128 ? (const void*)k_pcg_solve_coop3<T, NT, CPT, 4>
+                      : (const void*)k_pcg_solve_coop3<T, NT, CPT, 8>;
+}
+template <class T>
+const void* coop3_kernel(const Coop3Grid& c)
+{
+    return c.nt == 256 ? (c.cpt == 2 ? coop3_kernel<T, 256, 2>(c.G) : coop3_kernel<T, 256, 4>(c.G))
+           : c.cpt == 4 ? coop3_kernel<T, 512, 4>(c.G)
+                        : coop3_kernel<T, 448, 10>(c.G);
 }
 
 } // namespace
@@ -997,9 +1043,12 @@ size_t coop_xch_bytes(const Geo& g)
     return (size_t)cg.G * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
 }
 
-bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgState* st,
-                           void* xch, unsigned& seq, int max_its, hipStream_t s)
+template <class T>
+bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* xch,
+                           unsigned& seq, int max_its, hipStream_t s)
 {
+    if (std::is_same<T, float>::value && g.dim != 3)
+        throw CfError(CF_EINVAL, "the cooperative FP32 PCG is 3-D");
     if (!pcg_coop_fits(g))
         throw CfError(CF_EINVAL, "grid does not fit the cooperative PCG");
     if (max_its < 1)
@@ -1016,7 +1065,7 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
     Geo ga = g;
     CoopGrid cg;
     Coop3Grid c3;
-    double *xa = x, *ra = r, *pa = p;
+    T *xa = x, *ra = r, *pa = p;
     PcgState* sta = st;
     int ma = max_its;
     void* args[] = {&ga, &cg, &xa, &ra, &pa, &sta, &xc, &ma};
@@ -1027,9 +1076,7 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
         c3 = coop3_grid(g);
         args[1] = &c3;
         xc.halo = xc.part + (size_t)c3.G * 16;
-        fn = c3.nt == 256 ? (c3.cpt == 2 ? coop3_kernel<256, 2>(c3.G) : coop3_kernel<256, 4>(c3.G))
-             : c3.cpt == 4 ? coop3_kernel<512, 4>(c3.G)
-                           : coop3_kernel<448, 10>(c3.G);
+        fn = coop3_kernel<T>(c3);
         grid = dim3(c3.G * c3.every);
         block = dim3(c3.nt + kWave);
         lds = coop3_lds(c3);
@@ -1052,5 +1099,9 @@ bool launch_pcg_solve_coop(const Geo& g, double* x, double* r, double* p, PcgSta
     seq += 2u * (unsigned)max_its;
     return true;
 }
+template bool launch_pcg_solve_coop<double>(const Geo&, double*, double*, double*, PcgState*,
+                                            void*, unsigned&, int, hipStream_t);
+template bool launch_pcg_solve_coop<float>(const Geo&, float*, float*, float*, PcgState*, void*,
+                                           unsigned&, int, hipStream_t);
 
 } // namespace cfmi

@@ -296,6 +296,14 @@ int VelocityCorrector::runIterations(T* x, T* r, DevArray<T> (&p)[2], int& cur,
     readState(hs);
     if (hs.done)
         return hs.iter;
+    // FP32 here means inside a refined solve (an FP64 one tries this first)
+    if (std::is_same<T, float>::value && pcgGeo().dim == 3 && !_coop_off &&
+        pcg_coop_fits(pcgGeo())) {
+        const int its = runCoop<T>(x, r, p[cur].ptr, predict);
+        if (its >= 0)
+            return its;
+        readState(hs);
+    }
     const int it0 = hs.iter;
     const bool pairs = pcg_pairs_x<T>(pcgGeo());
     int launched = 0;
@@ -334,7 +342,9 @@ int VelocityCorrector::runPcg64(const double* b, double* x, double tol,
     RedBuf rb{_red_partials.ptr, _red_counter.ptr};
     launch_pcg_init64(pcgGeo(), b, x, _r.ptr, _st, tol, maxit, rb, _s);
     int cur = 0;
-    int its = !_coop_off && pcg_coop_fits(pcgGeo()) ? runCoop(x) : -1;
+    int its = -1;
+    if (!_coop_off && pcg_coop_fits(pcgGeo()))
+        its = runCoop<double>(x, _r.ptr, _p[0].ptr, _predict64);
     // the streaming kernels, or where a cooperative launch was refused, on
     // from the state it left (p[0] holds the current direction)
     if (its < 0)
@@ -351,16 +361,17 @@ int VelocityCorrector::runPcg64(const double* b, double* x, double tol,
 // runtime refuses a cooperative launch.
 constexpr int kCoopItsPerLaunch = 256;
 
-int VelocityCorrector::runCoop(double* x)
+template <class T>
+int VelocityCorrector::runCoop(T* x, T* r, T* p, int predict)
 {
     if (!_xch.ptr)
         _xch.alloc((int64_t)(coop_xch_bytes(pcgGeo()) + sizeof(double) - 1) / sizeof(double), _s);
     PcgState hs;
-    int its = _predict64 + 64 > kCoopItsPerLaunch ? _predict64 + 64 : kCoopItsPerLaunch;
+    int its = predict + 64 > kCoopItsPerLaunch ? predict + 64 : kCoopItsPerLaunch;
     for (;; its = kCoopItsPerLaunch) {
         const int t0 = _timer.begin(_s);
-        const bool ran = launch_pcg_solve_coop(pcgGeo(), x, _r.ptr, _p[0].ptr, _st, _xch.ptr,
-                                               _xch_seq, its, _s);
+        const bool ran = launch_pcg_solve_coop<T>(pcgGeo(), x, r, p, _st, _xch.ptr, _xch_seq, its,
+                                                  _s);
         _timer.end(t0, _s, TK_PCG_COOP, 0);
         if (!ran) {
             _timer.resolve(INT_MAX);

@@ -187,8 +187,9 @@ class VelocityCorrector
     int runIterations(T* x, T* r, DevArray<T> (&p)[2], int& cur, int predict,
                       int tk0);
     int runPcg64(const double* b, double* x, double tol, int maxit);
-    // the whole FP64 solve by the cooperative kernel (pcg_coop_fits)
-    int runCoop(double* x);
+    // iterations to the stop by the cooperative kernel (pcg_coop_fits)
+    template <class T>
+    int runCoop(T* x, T* r, T* p, int predict);
     void readState(PcgState& host);
     void readRefine();
     int& passPrediction(int pass);
