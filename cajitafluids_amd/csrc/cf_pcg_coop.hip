@@ -78,7 +78,9 @@ struct CoopGrid
 };
 
 // The strips' shape: 4 cells a lane of 256 lanes while that makes at most 64
-// strips, 4 of 512 up to 128 strips, else 10 of 448 (with the scalars' wave two
+// strips, 4 of 512 up to 128 strips and where that makes one of two (45^2
+// 3.9 -> 2.3 us an iteration; 3840 cells in one strip of 960 lanes gained 7%
+// over two to four, 4096 in one of 448 nothing), else 10 of 448 (with the scalars' wave two
 // waves a SIMD: 8 of 512 with it left 168 registers a lane, and spilled).
 // Fewer, larger strips shorten the exchanges and lengthen the strip's own
 // chain.  us per iteration at 4 of 256, 4 of 512 and 8 of 512 lanes, with the
@@ -99,6 +101,8 @@ CoopGrid coop_grid(const Geo& g)
         if (cg.R > g.n[1])
             cg.R = g.n[1];
         cg.G = cg.R > 0 ? (g.n[1] + cg.R - 1) / cg.R : INT_MAX;
+        if (cg.G > 1 && (int64_t)g.n[0] * g.n[1] <= 4 * 512 && cg.nt == 256)
+            continue;
         if (cg.G <= sh[2])
             break;
     }
@@ -990,7 +994,8 @@ Coop3Grid coop3_grid(const Geo& g)
             if (halo > kCoopHalo * nt || c.nwin >= 1 << 16 ||
                 coop3_lds(c) > 150 * 1024)
                 continue;
-            const double us = 2.0 * (1.3 + 0.1 * std::log2((double)G) + 0.006 * G) + 1.5 +
+            const double xch = G > 1 ? 1.3 + 0.1 * std::log2((double)G) + 0.006 * G : 0.15;
+            const double us = 2.0 * xch + 1.5 +
                               0.25 * (nt * cpt) / 256.0 + 1e-3 * halo / nt * 200.0 +
                               3.2e-6 * halo * G;
             if (us < cost) {
@@ -1090,7 +1095,11 @@ bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* x
         block = dim3(cg.nt + kWave);
         lds = coop_lds(g, cg);
     }
-    const hipError_t e = hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
+    // A lone workgroup waits for no other: an ordinary launch will do, which
+    // costs 20 us less (a 32^2 step 232 -> 211 us).
+    const hipError_t e =
+        grid.x == 1 ? hipLaunchKernel(fn, grid, block, args, lds, s)
+                    : hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
     if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
         (void)hipGetLastError(); // refused before anything ran
         return false;

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [
     ((32, 32), (1, 1)), ((33, 31), (0, 0)), ((31, 34), (0, 1)), ((5, 3), (0, 0)),
+    ((64, 32), (1, 1)), ((45, 45), (0, 0)), ((64, 33), (0, 1)),
     ((128, 256), (0, 0)), ((128, 257), (0, 1)), ((256, 256), (1, 0)), ((256, 257), (0, 0)),
     ((1024, 64), (0, 0)), ((1025, 40), (1, 1)), ((600, 600), (0, 0)), ((1200, 700), (0, 1)),
     ((2300, 30), (0, 0)),
