@@ -393,7 +393,7 @@ def advect_figures(cfg, avg_ms):
         out.update(flops_per_point=ADVECT_FLOPS_PER_POINT_3D_CUBIC,
                    tflops=round(tf, 2), fp64_peak_frac=round(tf / FP64_PEAK_TFLOPS, 4),
                    hbm_frac=round(out["gbs_unique"] / HBM_PEAK_GBS, 4),
-                   bound="gathers: 136 taps per point through L1/L2, three RK3 stages in sequence")
+                   bound="vector issue: velocity taps from an LDS window, three RK3 stages in sequence")
     return out
 
 

@@ -27,8 +27,8 @@
 // What bounds it: vector issue.  A block computes its overlap too (at 256^3
 // 1.8 cells per owned cell) and all its waves wait for each other at every
 // plane.  Measured, six launches before and two now: 256^3 level 0 in FP64
-// 400 -> 217 us (0.7 GB, 3.2 TB/s), 190 x 182 x 149 level 0 in FP32 130 -> 67
-// us, a 2-D level of 391 x 263 31 -> 14 us.  The first forms were slower than
+// 400 -> 202 us (0.7 GB, 3.5 TB/s), 190 x 182 x 149 level 0 in FP32 130 -> 66
+// us, a 2-D level of 391 x 263 31 -> 13 us.  The first forms were slower than
 // the six launches: rows at a wall on a path of their own (every wave of the
 // block waits for them at each plane: 175 us a leg), and loads in flight
 // copied at the loop's end (settle()).
