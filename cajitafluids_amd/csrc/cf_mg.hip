@@ -684,7 +684,8 @@ __device__ __forceinline__ void mg_coarsest_wave(const MgLev& L, const double* _
 // 0.3 us.  256^3 (levels of 16^3 and below): 24 us; with every cell's entries
 // computed in every sweep (an FP64 division, integer face counts), a parent's
 // eight residuals in one thread and 8^3 as the largest level it took 35.
-// 391 x 263 (49 x 33 and below): 56 -> 19; 190 x 182 x 149: 58 -> 19.
+// 391 x 263 (49 x 33 and below): 56 -> 19; 190 x 182 x 149: 58 -> 19.  With the
+// reads it starts with under way before the state's: 23, 18.8 and 16.7.
 struct TailCell
 {
     double diag, w, cx, cy, cz, b, x;
@@ -756,13 +757,25 @@ __device__ __forceinline__ void tail_each(int n, TailCell (&t)[kMgTailCells], F&
         }
 }
 
-__global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(const MgTail* __restrict__ T,
+__global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(MgTailTop top,
+                                                            const MgTail* __restrict__ T,
                                                             const PcgState* st)
 {
     extern __shared__ double lds[];
+    const int l0 = top.l0, last = top.last;
+    // what goes to LDS is on its way before the state is read
+    constexpr int W = sizeof(MgOpTab<double>) / sizeof(double);
+    const int n_op = (last - l0) * W, n_rest = top.n_all - top.n_top;
+    auto op_at = [&](int q) {
+        return reinterpret_cast<const double*>(&top.op[l0 + q / W].d) + q % W;
+    };
+    const double first_op = n_op > 0 ? *op_at(min((int)threadIdx.x, n_op - 1)) : 0.0;
+    const MgTailInfo first_info =
+        top.info[min(top.n_top + (int)threadIdx.x, top.n_all - 1)];
+    asm volatile("" ::: "memory");
     if (st->done)
         return;
-    const int l0 = T->l0, last = T->last, nu = T->nu, coarse = T->coarse;
+    const int nu = T->nu, coarse = T->coarse;
     const int dim = T->lev[l0].dim;
     const double alpha = T->lev[l0].alpha;
     // the vectors of level l: X and T with their slot of -0 ahead, and B
@@ -772,17 +785,15 @@ __global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(const MgTail* __rest
     MgOpTab<double>* ops = reinterpret_cast<MgOpTab<double>*>(lds + T->off[last + 1]);
     // the cells' MgTailInfo: level l0's in memory, the others' copied to LDS
     MgTailInfo* infos = reinterpret_cast<MgTailInfo*>(ops + (last - l0));
-    const int n_top = T->lev[l0].ncell, n_all = T->info_at[last + 1];
+    const int n_top = top.n_top;
     auto info = [&](int l, int id) -> MgTailInfo {
-        return l == l0 ? T->info[id] : infos[T->info_at[l] - n_top + id];
+        return l == l0 ? top.info[id] : infos[T->info_at[l] - n_top + id];
     };
     {
-        for (int q = threadIdx.x; q < n_all - n_top; q += kMgTailThreads)
-            infos[q] = T->info[n_top + q];
-        constexpr int W = sizeof(MgOpTab<double>) / sizeof(double);
-        for (int q = threadIdx.x; q < (last - l0) * W; q += kMgTailThreads)
-            reinterpret_cast<double*>(ops)[q] =
-                reinterpret_cast<const double*>(&T->op[l0 + q / W].d)[q % W];
+        for (int q = threadIdx.x; q < n_rest; q += kMgTailThreads)
+            infos[q] = q < kMgTailThreads ? first_info : top.info[n_top + q];
+        for (int q = threadIdx.x; q < n_op; q += kMgTailThreads)
+            reinterpret_cast<double*>(ops)[q] = q < kMgTailThreads ? first_op : *op_at(q);
         if ((int)threadIdx.x < last - l0) {
             X(l0 + threadIdx.x)[-1] = -0.0;
             Tv(l0 + threadIdx.x)[-1] = -0.0;
@@ -807,13 +818,11 @@ __global__ __launch_bounds__(kMgTailThreads) void k_mg_tail(const MgTail* __rest
         if (small && !wave0)
             break; // wave 0 goes on alone
         double *x = X(l), *u = Tv(l), *bv = Bv(l);
-        const double* bg = T->B[l0];
         const int fn0 = l > l0 ? T->lev[l - 1].n[0] : 0;
         const int fn01 = l > l0 ? fn0 * T->lev[l - 1].n[1] : 0;
         tail_each(n, t, [&](TailCell& c, int id) {
-            if (l == l0) {
-                c.b = bg[id];
-            }
+            if (l == l0)
+                c.b = top.b[id];
             const MgTailInfo f = info(l, id);
             if (l > l0)
                 c.b = tail_children(f, mg_tail_residual(X(l - 1), Tv(l - 1), nu), fn0, fn01);
@@ -1230,9 +1239,10 @@ void launch_mg_resrestrict(const MgLev& F, const MgLev& C, const double* x, cons
                        bc, st);
 }
 
-void launch_mg_tail(const MgTail* t_dev, size_t lds_bytes, const PcgState* st, hipStream_t s)
+void launch_mg_tail(const MgTailTop& top, const MgTail* t_dev, size_t lds_bytes,
+                    const PcgState* st, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kMgTailThreads), lds_bytes, s, t_dev, st);
+    hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kMgTailThreads), lds_bytes, s, top, t_dev, st);
 }
 
 void launch_mgpcg_init(const Geo& g, const double* b, double* x, double* r, PcgState* st,

@@ -104,6 +104,16 @@ struct MgTail
     int info_at[kMgMaxLevels + 1];
 };
 
+// What k_mg_tail starts with, by value: the top level's right-hand side and
+// cells, and what it copies to LDS.
+struct MgTailTop
+{
+    int l0, last, n_top, n_all; // cells of level l0, MgTailInfo in all
+    const double* b;
+    const MgTailInfo* info; // MgTail::info
+    const MgOp* op;
+};
+
 // Which of a level's two vectors k_mg_tail's downward leg leaves the residual
 // in: x = w b in X, then nu - 1 sweeps and the residual, alternating.  The
 // upward leg's nu sweeps from there end in X.
@@ -212,7 +222,8 @@ void launch_mg_smooth(const MgLev& L, int src, const double* xi, const double* b
 void launch_mg_resrestrict(const MgLev& F, const MgLev& C, const double* x, const double* b,
                            double* bc, const PcgState* st, hipStream_t s);
 // One workgroup runs the V-cycle of levels t->l0 .. t->last in lds_bytes of LDS.
-void launch_mg_tail(const MgTail* t_dev, size_t lds_bytes, const PcgState* st, hipStream_t s);
+void launch_mg_tail(const MgTailTop& top, const MgTail* t_dev, size_t lds_bytes,
+                    const PcgState* st, hipStream_t s);
 
 // MG-PCG: r = b, x = 0, ||b|| (sets st->mg); and rho / beta from r.z.
 void launch_mgpcg_init(const Geo& g, const double* b, double* x, double* r,

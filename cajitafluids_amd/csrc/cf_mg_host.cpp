@@ -38,6 +38,7 @@ struct Multigrid::Buffers
     std::vector<std::unique_ptr<DevArray<double>>> vec;
     std::vector<double*> X, T, B, res;
     MgTail* tail = nullptr; // device copy
+    MgTailTop top{};
     MgTailInfo* info = nullptr; // its cells, device
     MgOp* op = nullptr;     // operator tables of the fused levels, device
     ~Buffers()
@@ -265,6 +266,8 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
                               hipMemcpyHostToDevice, s));
         CF_HIP(hipStreamSynchronize(s)); // info is this block's
         h.info = B.info;
+        B.top = MgTailTop{_tail0, last, _lev[_tail0].ncell, (int)info.size(), B.B[_tail0], B.info,
+                          B.op};
         CF_HIP(hipMalloc(&p, sizeof(MgTail)));
         B.tail = (MgTail*)p;
         CF_HIP(hipMemcpyAsync(B.tail, &h, sizeof(MgTail), hipMemcpyHostToDevice, s));
@@ -559,7 +562,7 @@ const void* Multigrid::cycle(const double* r, PcgState* st, RedBuf rb, bool f32,
         }
         resrestrict(l, x, b, st);
     }
-    launch_mg_tail(B.tail, _tail_lds, st, _s);
+    launch_mg_tail(B.top, B.tail, _tail_lds, st, _s);
     // up: the first post-sweep reads the coarse correction; on level 0 the
     // last sweep also reduces r.z
     const bool pre_odd = (_nu >= 2 ? _nu - 2 : 0) & 1;
