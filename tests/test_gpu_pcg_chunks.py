@@ -1,6 +1,8 @@
 """The z chunks of the 3-D PCG tiles: grids whose chunks are one, two or
 three planes deep, end in a shorter chunk, or fill the GPU unevenly, against
-the oracle bit for bit (truncated solves: every iterate, not the limit)."""
+the oracle bit for bit (truncated solves: every iterate, not the limit).
+Grids of up to about 100^3 with rows of at most 1024 cells run cooperatively;
+the longer rows and the largest grid run the tiles."""
 import numpy as np
 import pytest
 
@@ -14,7 +16,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,periodic", [
     ((7, 5, 1), (0, 0, 0)), ((9, 6, 2), (0, 0, 0)), ((33, 17, 3), (1, 0, 0)),
     ((65, 15, 7), (0, 1, 1)), ((45, 52, 61), (0, 0, 0)), ((129, 33, 10), (1, 1, 0)),
-    ((150, 141, 83), (0, 0, 1))])
+    ((150, 141, 83), (0, 0, 1)), ((1025, 5, 1), (0, 0, 0)), ((1030, 17, 2), (1, 0, 0)),
+    ((1100, 15, 7), (0, 1, 1)), ((1026, 33, 20), (1, 1, 0))])
 def test_pcg_3d_chunk_depths(oracle_mod, n, periodic, precision):
     from cajitafluids_amd import _lib
     from cajitafluids_amd.solver import Solver
