@@ -132,14 +132,16 @@ struct AdvWin
     double mid[3], half[3];
 };
 
-// A block-uniform value, moved to scalar registers.
+// A block-uniform value, moved to scalar registers (the empty asm hides that
+// it is uniform, or the move is dropped).  The lane reads are the compiler's,
+// with the wait states they need after the write of what they read and before
+// their result's use.
 __device__ __forceinline__ double uniform(double v)
 {
-    const long long b = __double_as_longlong(v);
-    unsigned lo, hi;
-    asm("v_readfirstlane_b32 %0, %1" : "=s"(lo) : "v"((unsigned)b));
-    asm("v_readfirstlane_b32 %0, %1" : "=s"(hi) : "v"((unsigned)(b >> 32)));
-    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    asm("" : "+v"(lo), "+v"(hi));
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(hi),
+                            __builtin_amdgcn_readfirstlane(lo));
 }
 
 // 8 bytes at a 32-bit byte offset from a uniform pointer.
