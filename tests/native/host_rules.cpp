@@ -1,0 +1,34 @@
+// Prints the library's host-side choices for a case, for tests/test_host_rules.py.
+//   host_rules leg DIM N0 N1 N2 P0 P1 P2 NU F32 BOXES: waves of the block in
+//     which a multigrid level of N cells with periodic axes P runs its legs
+//     (0: sweep by sweep); BOXES: a level whose couplings differ.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+#include "cf_mg.hpp"
+
+using namespace cfmi;
+
+static int leg(char** a)
+{
+    MgLev L{};
+    L.dim = std::atoi(a[0]);
+    for (int d = 0; d < 3; ++d) {
+        L.n[d] = std::atoi(a[1 + d]);
+        L.periodic[d] = std::atoi(a[4 + d]);
+        L.coarsen[d] = d < L.dim && L.n[d] > 2;
+    }
+    MgFused f{};
+    const bool fused = mg_fused_level(L, std::atoi(a[7]), std::atoi(a[8]) != 0,
+                                      std::atoi(a[9]) ? 0.0 : -1.0, f);
+    std::printf("%d\n", fused ? f.waves : 0);
+    return 0;
+}
+
+int main(int argc, char** argv)
+{
+    if (argc == 12 && !std::strcmp(argv[1], "leg"))
+        return leg(argv + 2);
+    return 2;
+}

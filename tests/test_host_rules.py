@@ -1,0 +1,38 @@
+"""The rules by which the library chooses kernels on the host, called on the
+CPU (tests/native/host_rules.cpp against the built library): the grids of the
+GPU tests run the kernels that those tests are for."""
+import os
+import subprocess
+
+import pytest
+
+import test_gpu_mg_waves as waves
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("native") / "host_rules")
+    lib = os.path.join(REPO, "cajitafluids_amd")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(REPO, "include"), "-I" + os.path.join(lib, "csrc"),
+                    "-o", exe, os.path.join(REPO, "tests", "native", "host_rules.cpp"),
+                    "-L" + lib, "-lcfmi", "-L/opt/rocm/lib", "-lamdhip64",
+                    "-Wl,-rpath," + lib + ":/opt/rocm/lib"], check=True)
+
+    def call(*args):
+        out = subprocess.run([exe, *map(str, args)], check=True, capture_output=True, text=True)
+        return [int(v) for v in out.stdout.split()]
+
+    return call
+
+
+@pytest.mark.parametrize("n,periodic,precision,nu,want", waves.CASES)
+def test_leg_waves(rules, n, periodic, precision, nu, want):
+    level = list(n)
+    for l, w in enumerate(want):
+        boxes = l > 0 and any(m % 2 for m in n)
+        f32 = precision == waves.K.FP32_REFINED and not boxes
+        assert rules("leg", 3, *level, *periodic, nu, int(f32), int(boxes)) == [w], level
+        level = [(m + 1) // 2 for m in level]
