@@ -123,22 +123,58 @@ inline bool pcg_pairs_x(const Geo& g)
 // partials buffer).
 int reduction_blocks_max(const Geo& g);
 
-// Jacobi-PCG iterations (FP64, or on 3-D grids FP32) in one cooperative launch of one workgroup per
-// strip of rows (2-D) or pencil of x-rows (3-D), until the state's stop test or `max_its`
-// iterations of this launch (x, r and the direction p are read at the start
-// and written back at the end, so launches chain).  The same x, r, direction
-// and state bits as the dir_spmv / update pair.  pcg_coop_fits: the grid
-// qualifies (at most 256 strips or pencils of whole rows and 4096 cells);
-// xch: coop_xch_bytes(g) bytes of device memory, zero at first; seq: the last
-// exchange number used there (0 at first), advanced by the call.  A launch that waited too
-// long for another workgroup sets PcgState::stalled.  Returns false when the
-// runtime refuses the cooperative launch (the workgroups cannot all be
-// resident, or the device has no cooperative launch); nothing ran then.
-bool pcg_coop_fits(const Geo& g);
-size_t coop_xch_bytes(const Geo& g);
+// Jacobi-PCG iterations (FP64, or on 3-D grids FP32) in one cooperative launch
+// of one workgroup per strip of rows (2-D) or pencil of x-rows (3-D), until the
+// state's stop test or `max_its` iterations of this launch (x, r and the
+// direction p are read at the start and written back at the end, so launches
+// chain).  The same x, r, direction and state bits as the dir_spmv / update
+// pair.
+
+// A 2-D grid's strips: R rows each, G of them; window row pitch e0 = n0 + 2
+// (window index of strip-relative cell (i, jj), halo rows jj = -1 and
+// jj = R: (i+1) + e0 (jj+1)).
+struct CoopGrid
+{
+    int G, R, e0, nwin;
+    int c00; // padded index of owned cell (0, 0)
+    int px;
+    int nt, cpt; // lanes per workgroup and cells per lane
+    int every;   // the strips are the launch's blocks 0, every, 2 every, ...
+};
+
+// A 3-D grid's pencils: by x bz x-rows each.
+struct Coop3Grid
+{
+    int G, by, bz, gy; // pencils, their rows along y and z, pencils along y
+    int e0, e1, nwin;  // window pitches (x row, plane) and size
+    int c00, px;       // padded index of owned cell (0, 0, 0), pitches
+    int64_t pxy;
+    int nt, cpt, every;
+};
+
+// How a grid is split.  It depends on the geometry alone, and a 3-D grid's
+// comes from a search over the pencils' shapes that takes the host 11 to 17
+// us: a solver makes it once (made anew by every launch, three times over, it
+// kept the GPU waiting in each pass of a refined solve).
+struct CoopPlan
+{
+    int groups = 0; // workgroups; 0: the grid does not fit
+    CoopGrid strips{};
+    Coop3Grid pencils{};
+    size_t lds = 0; // bytes of a workgroup
+    size_t xch = 0; // bytes of the exchange buffer
+};
+CoopPlan coop_plan(const Geo& g);
+
+// plan: coop_plan's of a grid that fits; xch: plan.xch bytes of device memory,
+// zero at first; seq: the last exchange number used there (0 at first),
+// advanced by the call.  A launch that waited too long for another workgroup
+// sets PcgState::stalled.  Returns false when the runtime refuses the
+// cooperative launch (the workgroups cannot all be resident, or the device has
+// no cooperative launch); nothing ran then.
 template <class T>
-bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* xch,
-                           unsigned& seq, int max_its, hipStream_t s);
+bool launch_pcg_solve_coop(const Geo& g, const CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
+                           void* xch, unsigned& seq, int max_its, hipStream_t s);
 
 // FP32-inner / FP64-outer defect correction.  The host runs the outer loop
 // from the device-computed norms (one read-back per pass).

@@ -65,18 +65,6 @@ constexpr int kCoopMaxGroups = 256;
 constexpr int kCoopCells = 4096; // of a strip or pencil at most
 constexpr unsigned kCoopSpin = 1u << 22; // polls (about 1 us each) before a wait counts as stalled
 
-// Strip layout: R rows per strip, G strips; window row pitch e0 = n0 + 2
-// (window index of strip-relative cell (i, jj), halo rows jj = -1 and
-// jj = R: (i+1) + e0 (jj+1)).
-struct CoopGrid
-{
-    int G, R, e0, nwin;
-    int c00; // padded index of owned cell (0, 0)
-    int px;
-    int nt, cpt; // lanes per workgroup and cells per lane
-    int every;   // the strips are the launch's blocks 0, every, 2 every, ...
-};
-
 // The strips' shape: 4 cells a lane of 256 lanes while that makes at most 64
 // strips, 4 of 512 up to 128 strips and where that makes one of two (45^2
 // 3.9 -> 2.3 us an iteration; 3840 cells in one strip of 960 lanes gained 7%
@@ -641,14 +629,6 @@ const void* coop_kernel(int G)
 // polls that place), so no pencil needs to know which one owns its halo.  A
 // halo cell's r stays in its lane's registers from the poll to the next
 // direction.  The wave that gathers the partials has no halo cells.
-struct Coop3Grid
-{
-    int G, by, bz, gy; // pencils, their rows along y and z, pencils along y
-    int e0, e1, nwin;  // window pitches (x row, plane) and size
-    int c00, px;       // padded index of owned cell (0, 0, 0), pitches
-    int64_t pxy;
-    int nt, cpt, every;
-};
 constexpr int kCoopHalo = 8; // halo cells per lane at most
 
 // A bit mask the compiler re-reads: its bits' tests are not all kept as lane
@@ -1028,78 +1008,74 @@ const void* coop3_kernel(const Coop3Grid& c)
 
 } // namespace
 
-bool pcg_coop_fits(const Geo& g)
+CoopPlan coop_plan(const Geo& g)
 {
-    if (g.dim == 3)
-        return coop3_grid(g).G > 0;
-    const CoopGrid cg = coop_grid(g);
-    if (cg.G > kCoopMaxGroups)
-        return false;
-    // window indices fit the slot word's 16 bits
-    return cg.nwin < (1 << 16) && coop_lds(g, cg) <= 128 * 1024;
-}
-
-size_t coop_xch_bytes(const Geo& g)
-{
-    if (g.dim == 3)
-        return ((size_t)coop3_grid(g).G * 16 + 2 * (size_t)g.n[0] * g.n[1] * g.n[2]) *
-               sizeof(Word);
-    const CoopGrid cg = coop_grid(g);
-    return (size_t)cg.G * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
+    CoopPlan c;
+    if (g.dim == 3) {
+        c.pencils = coop3_grid(g);
+        c.groups = c.pencils.G;
+        c.lds = coop3_lds(c.pencils);
+        c.xch = ((size_t)c.groups * 16 + 2 * (size_t)g.n[0] * g.n[1] * g.n[2]) * sizeof(Word);
+    } else {
+        c.strips = coop_grid(g);
+        if (c.strips.G > kCoopMaxGroups)
+            return c;
+        c.lds = coop_lds(g, c.strips);
+        // window indices fit the slot word's 16 bits
+        if (c.strips.nwin >= (1 << 16) || c.lds > 128 * 1024)
+            return c;
+        c.groups = c.strips.G;
+        c.xch = (size_t)c.groups * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
+    }
+    return c;
 }
 
 template <class T>
-bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* xch,
-                           unsigned& seq, int max_its, hipStream_t s)
+bool launch_pcg_solve_coop(const Geo& g, const CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
+                           void* xch, unsigned& seq, int max_its, hipStream_t s)
 {
     if (std::is_same<T, float>::value && g.dim != 3)
         throw CfError(CF_EINVAL, "the cooperative FP32 PCG is 3-D");
-    if (!pcg_coop_fits(g))
+    if (plan.groups < 1)
         throw CfError(CF_EINVAL, "grid does not fit the cooperative PCG");
     if (max_its < 1)
         throw CfError(CF_EINVAL, "the cooperative PCG runs at least one iteration per launch");
     // a word is new when it carries its exchange's number: the numbers go on
     // from launch to launch, and before they wrap the buffer is cleared
     if (seq > 0xffffffffu - 2u * (unsigned)max_its - 2u) {
-        CF_HIP(hipMemsetAsync(xch, 0, coop_xch_bytes(g), s));
+        CF_HIP(hipMemsetAsync(xch, 0, plan.xch, s));
         seq = 0;
     }
     CoopXch xc;
     xc.part = (Word*)xch;
+    xc.halo = xc.part + (size_t)plan.groups * 16;
     xc.seq0 = seq;
     Geo ga = g;
-    CoopGrid cg;
-    Coop3Grid c3;
+    CoopGrid cg = plan.strips;
+    Coop3Grid c3 = plan.pencils;
     T *xa = x, *ra = r, *pa = p;
     PcgState* sta = st;
     int ma = max_its;
     void* args[] = {&ga, &cg, &xa, &ra, &pa, &sta, &xc, &ma};
     const void* fn;
     dim3 grid, block;
-    size_t lds;
     if (g.dim == 3) {
-        c3 = coop3_grid(g);
         args[1] = &c3;
-        xc.halo = xc.part + (size_t)c3.G * 16;
         fn = coop3_kernel<T>(c3);
         grid = dim3(c3.G * c3.every);
         block = dim3(c3.nt + kWave);
-        lds = coop3_lds(c3);
     } else {
-        cg = coop_grid(g);
-        xc.halo = xc.part + (size_t)cg.G * 16;
         fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
              : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
                            : coop_kernel<448, 10>(cg.G);
         grid = dim3(cg.G * cg.every);
         block = dim3(cg.nt + kWave);
-        lds = coop_lds(g, cg);
     }
     // A lone workgroup waits for no other: an ordinary launch will do, which
     // costs 20 us less (a 32^2 step 232 -> 211 us).
     const hipError_t e =
-        grid.x == 1 ? hipLaunchKernel(fn, grid, block, args, lds, s)
-                    : hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)lds, s);
+        grid.x == 1 ? hipLaunchKernel(fn, grid, block, args, plan.lds, s)
+                    : hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)plan.lds, s);
     if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
         (void)hipGetLastError(); // refused before anything ran
         return false;
@@ -1108,9 +1084,9 @@ bool launch_pcg_solve_coop(const Geo& g, T* x, T* r, T* p, PcgState* st, void* x
     seq += 2u * (unsigned)max_its;
     return true;
 }
-template bool launch_pcg_solve_coop<double>(const Geo&, double*, double*, double*, PcgState*,
-                                            void*, unsigned&, int, hipStream_t);
-template bool launch_pcg_solve_coop<float>(const Geo&, float*, float*, float*, PcgState*, void*,
-                                           unsigned&, int, hipStream_t);
+template bool launch_pcg_solve_coop<double>(const Geo&, const CoopPlan&, double*, double*, double*,
+                                            PcgState*, void*, unsigned&, int, hipStream_t);
+template bool launch_pcg_solve_coop<float>(const Geo&, const CoopPlan&, float*, float*, float*,
+                                           PcgState*, void*, unsigned&, int, hipStream_t);
 
 } // namespace cfmi

@@ -183,7 +183,7 @@ void step(ProblemManager& pm, hipStream_t s, KernelTimer& timer)
 // ---- VelocityCorrector -----------------------------------------------------------
 VelocityCorrector::VelocityCorrector(ProblemManager& pm, const cf_config& cfg,
                                      hipStream_t s, KernelTimer& timer)
-    : _pm(pm), _cfg(cfg), _s(s), _timer(timer), _g(pm.mesh().geo())
+    : _pm(pm), _cfg(cfg), _s(s), _timer(timer), _g(pm.mesh().geo()), _coop(coop_plan(_g))
 {
     const int64_t n = _g.total;
     _g_unit = _g;
@@ -298,7 +298,7 @@ int VelocityCorrector::runIterations(T* x, T* r, DevArray<T> (&p)[2], int& cur,
         return hs.iter;
     // FP32 here means inside a refined solve (an FP64 one tries this first)
     if (std::is_same<T, float>::value && pcgGeo().dim == 3 && !_coop_off &&
-        pcg_coop_fits(pcgGeo())) {
+        _coop.groups > 0) {
         const int its = runCoop<T>(x, r, p[cur].ptr, predict);
         if (its >= 0)
             return its;
@@ -343,7 +343,7 @@ int VelocityCorrector::runPcg64(const double* b, double* x, double tol,
     launch_pcg_init64(pcgGeo(), b, x, _r.ptr, _st, tol, maxit, rb, _s);
     int cur = 0;
     int its = -1;
-    if (!_coop_off && pcg_coop_fits(pcgGeo()))
+    if (!_coop_off && _coop.groups > 0)
         its = runCoop<double>(x, _r.ptr, _p[0].ptr, _predict64);
     // the streaming kernels, or where a cooperative launch was refused, on
     // from the state it left (p[0] holds the current direction)
@@ -365,13 +365,13 @@ template <class T>
 int VelocityCorrector::runCoop(T* x, T* r, T* p, int predict)
 {
     if (!_xch.ptr)
-        _xch.alloc((int64_t)(coop_xch_bytes(pcgGeo()) + sizeof(double) - 1) / sizeof(double), _s);
+        _xch.alloc((int64_t)(_coop.xch + sizeof(double) - 1) / sizeof(double), _s);
     PcgState hs;
     int its = predict + 64 > kCoopItsPerLaunch ? predict + 64 : kCoopItsPerLaunch;
     for (;; its = kCoopItsPerLaunch) {
         const int t0 = _timer.begin(_s);
-        const bool ran = launch_pcg_solve_coop<T>(pcgGeo(), x, r, p, _st, _xch.ptr, _xch_seq, its,
-                                                  _s);
+        const bool ran = launch_pcg_solve_coop<T>(pcgGeo(), _coop, x, r, p, _st, _xch.ptr,
+                                                  _xch_seq, its, _s);
         _timer.end(t0, _s, TK_PCG_COOP, 0);
         if (!ran) {
             _timer.resolve(INT_MAX);

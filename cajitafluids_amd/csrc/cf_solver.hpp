@@ -187,7 +187,7 @@ class VelocityCorrector
     int runIterations(T* x, T* r, DevArray<T> (&p)[2], int& cur, int predict,
                       int tk0);
     int runPcg64(const double* b, double* x, double tol, int maxit);
-    // iterations to the stop by the cooperative kernel (pcg_coop_fits)
+    // iterations to the stop by the cooperative kernel (_coop.groups > 0)
     template <class T>
     int runCoop(T* x, T* r, T* p, int predict);
     void readState(PcgState& host);
@@ -200,6 +200,7 @@ class VelocityCorrector
     hipStream_t _s;
     KernelTimer& _timer;
     const Geo& _g;
+    CoopPlan _coop; // of the cooperative PCG
     DevArray<double> _lhs, _rhs, _r, _p[2];
     DevArray<float> _d32, _r32, _p32[2];
     DevArray<double> _red_partials, _scratch;

@@ -2,13 +2,23 @@
 //   host_rules leg DIM N0 N1 N2 P0 P1 P2 NU F32 BOXES: waves of the block in
 //     which a multigrid level of N cells with periodic axes P runs its legs
 //     (0: sweep by sweep); BOXES: a level whose couplings differ.
+//   host_rules coop DIM N0 N1 N2: workgroups of the cooperative solve (0: the
+//     grid does not fit) and their LDS bytes.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 
+#include <type_traits>
+
 #include "cf_mg.hpp"
 
 using namespace cfmi;
+
+// The launch takes the plan that its caller keeps, and makes none.
+static_assert(std::is_same<decltype(&launch_pcg_solve_coop<double>),
+                           bool (*)(const Geo&, const CoopPlan&, double*, double*, double*,
+                                    PcgState*, void*, unsigned&, int, hipStream_t)>::value,
+              "a launch of the cooperative solve is given its plan");
 
 static int leg(char** a)
 {
@@ -26,9 +36,25 @@ static int leg(char** a)
     return 0;
 }
 
+static int coop(char** a)
+{
+    Geo g{};
+    g.dim = std::atoi(a[0]);
+    g.h = 1;
+    for (int d = 0; d < 3; ++d)
+        g.n[d] = std::atoi(a[1 + d]);
+    g.px = g.n[0] + 3;
+    g.py = g.n[1] + 3;
+    const CoopPlan c = coop_plan(g);
+    std::printf("%d %zu\n", c.groups, c.lds);
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
     if (argc == 12 && !std::strcmp(argv[1], "leg"))
         return leg(argv + 2);
+    if (argc == 6 && !std::strcmp(argv[1], "coop"))
+        return coop(argv + 2);
     return 2;
 }

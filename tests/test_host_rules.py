@@ -36,3 +36,21 @@ def test_leg_waves(rules, n, periodic, precision, nu, want):
         f32 = precision == waves.K.FP32_REFINED and not boxes
         assert rules("leg", 3, *level, *periodic, nu, int(f32), int(boxes)) == [w], level
         level = [(m + 1) // 2 for m in level]
+
+
+@pytest.mark.parametrize("dim,n,fits", [
+    (2, (1, 1, 1), True), (2, (32, 32, 1), True), (2, (1024, 1024, 1), True),
+    (2, (2337, 256, 1), True), (2, (2338, 10, 1), False), (2, (1200, 1200, 1), False),
+    (3, (1, 1, 1), True), (3, (45, 52, 61), True), (3, (100, 100, 100), True),
+    (3, (682, 20, 20), True), (3, (683, 2, 2), False), (3, (128, 128, 128), False),
+    (3, (256, 256, 256), False)])
+def test_coop_plan(rules, dim, n, fits):
+    """A plan is made from the geometry alone, without a GPU, and handed to the
+    launches; what fits: at most 256 workgroups of 4096 cells, whole x-rows."""
+    groups, lds = rules("coop", dim, *n)
+    cells = n[0] * n[1] * n[2]
+    if fits:
+        assert (cells + 4095) // 4096 <= groups <= 256
+        assert 0 < lds <= 150 * 1024
+    else:
+        assert groups == 0
