@@ -166,14 +166,30 @@ struct CoopPlan
 };
 CoopPlan coop_plan(const Geo& g);
 
-// plan: coop_plan's of a grid that fits; xch: plan.xch bytes of device memory,
+// launch(every): whether the runtime took a launch of the workgroups on every
+// `every`-th block.  It counts the idle blocks between them as if they had to
+// be resident too, so a device (a partition) with fewer compute units may
+// refuse those and hold the workgroups alone: 128^2 asks for 128 blocks, of
+// which 32 units hold 96, for its 16.  Then every = 1 from there on.
+template <class F>
+bool coop_spread(int& every, F&& launch)
+{
+    if (launch(every))
+        return true;
+    if (every == 1)
+        return false;
+    every = 1;
+    return launch(every);
+}
+
+// plan: coop_plan's of a grid that fits (the call may change its spread); xch: plan.xch bytes of device memory,
 // zero at first; seq: the last exchange number used there (0 at first),
 // advanced by the call.  A launch that waited too long for another workgroup
 // sets PcgState::stalled.  Returns false when the runtime refuses the
 // cooperative launch (the workgroups cannot all be resident, or the device has
 // no cooperative launch); nothing ran then.
 template <class T>
-bool launch_pcg_solve_coop(const Geo& g, const CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
+bool launch_pcg_solve_coop(const Geo& g, CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
                            void* xch, unsigned& seq, int max_its, hipStream_t s);
 
 // FP32-inner / FP64-outer defect correction.  The host runs the outer loop

@@ -1031,7 +1031,7 @@ CoopPlan coop_plan(const Geo& g)
 }
 
 template <class T>
-bool launch_pcg_solve_coop(const Geo& g, const CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
+bool launch_pcg_solve_coop(const Geo& g, CoopPlan& plan, T* x, T* r, T* p, PcgState* st,
                            void* xch, unsigned& seq, int max_its, hipStream_t s)
 {
     if (std::is_same<T, float>::value && g.dim != 3)
@@ -1058,35 +1058,43 @@ bool launch_pcg_solve_coop(const Geo& g, const CoopPlan& plan, T* x, T* r, T* p,
     int ma = max_its;
     void* args[] = {&ga, &cg, &xa, &ra, &pa, &sta, &xc, &ma};
     const void* fn;
-    dim3 grid, block;
+    int* every;
+    int lanes;
     if (g.dim == 3) {
         args[1] = &c3;
         fn = coop3_kernel<T>(c3);
-        grid = dim3(c3.G * c3.every);
-        block = dim3(c3.nt + kWave);
+        every = &plan.pencils.every;
+        lanes = c3.nt;
     } else {
         fn = cg.nt == 256 ? coop_kernel<256, 4>(cg.G)
              : cg.cpt == 4 ? coop_kernel<512, 4>(cg.G)
                            : coop_kernel<448, 10>(cg.G);
-        grid = dim3(cg.G * cg.every);
-        block = dim3(cg.nt + kWave);
+        every = &plan.strips.every;
+        lanes = cg.nt;
     }
-    // A lone workgroup waits for no other: an ordinary launch will do, which
-    // costs 20 us less (a 32^2 step 232 -> 211 us).
-    const hipError_t e =
-        grid.x == 1 ? hipLaunchKernel(fn, grid, block, args, plan.lds, s)
-                    : hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)plan.lds, s);
-    if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
-        (void)hipGetLastError(); // refused before anything ran
+    const bool ran = coop_spread(*every, [&](int spread) {
+        cg.every = c3.every = spread;
+        const dim3 grid(plan.groups * spread), block(lanes + kWave);
+        // A lone workgroup waits for no other: an ordinary launch will do,
+        // which costs 20 us less (a 32^2 step 232 -> 211 us).
+        const hipError_t e =
+            grid.x == 1 ? hipLaunchKernel(fn, grid, block, args, plan.lds, s)
+                        : hipLaunchCooperativeKernel(fn, grid, block, args, (unsigned)plan.lds, s);
+        if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported) {
+            (void)hipGetLastError(); // refused before anything ran
+            return false;
+        }
+        CF_HIP(e);
+        return true;
+    });
+    if (!ran)
         return false;
-    }
-    CF_HIP(e);
     seq += 2u * (unsigned)max_its;
     return true;
 }
-template bool launch_pcg_solve_coop<double>(const Geo&, const CoopPlan&, double*, double*, double*,
+template bool launch_pcg_solve_coop<double>(const Geo&, CoopPlan&, double*, double*, double*,
                                             PcgState*, void*, unsigned&, int, hipStream_t);
-template bool launch_pcg_solve_coop<float>(const Geo&, const CoopPlan&, float*, float*, float*,
+template bool launch_pcg_solve_coop<float>(const Geo&, CoopPlan&, float*, float*, float*,
                                            PcgState*, void*, unsigned&, int, hipStream_t);
 
 } // namespace cfmi

@@ -54,3 +54,17 @@ def test_coop_plan(rules, dim, n, fits):
         assert 0 < lds <= 150 * 1024
     else:
         assert groups == 0
+
+
+@pytest.mark.parametrize("dim,n,blocks,want", [
+    (2, (128, 128, 1), 512, [1, 128, 1, 1, 128, 1]),  # 16 strips on every eighth block
+    (2, (128, 128, 1), 96, [1, 16, 2, 1, 16, 1]),
+    (2, (128, 128, 1), 15, [0, 16, 2, 0, 16, 1]),
+    (2, (32, 32, 1), 1, [1, 1, 1, 1, 1, 1]),
+    (3, (20, 20, 20), 1, [0, 16, 2, 0, 16, 1]),
+    (3, (20, 20, 20), 16, [1, 16, 2, 1, 16, 1]),
+])
+def test_coop_spread(rules, dim, n, blocks, want):
+    """A device that does not hold the idle blocks between the workgroups still
+    runs the solve if it holds the workgroups."""
+    assert rules("spread", dim, *n, blocks) == want
