@@ -2,11 +2,19 @@
 the library links).
 
 Disassembles the gfx950 code objects of a file built here (its .hip_fatbin
-section) and fails on lane reads too close to their neighbours: the hardware
-needs one wait state between a vector instruction that writes a VGPR and the
-v_readfirstlane / v_readlane that reads it, and two between that lane read
-and a vector instruction that reads its SGPR.  The compiler inserts them
-around its own instructions, not around those of an inline asm.
+section) and fails on
+
+- lane reads too close to their neighbours: the hardware needs one wait state
+  between a vector instruction that writes a VGPR and the v_readfirstlane /
+  v_readlane that reads it, and two between that lane read and a vector
+  instruction that reads its SGPR.  The compiler inserts them around its own
+  instructions, not around those of an inline asm.
+- register moves before a join's lanes are back: where lanes that took a
+  branch meet those that skipped it, the block opens with `s_or_b64 exec,
+  exec, ...`.  Under register pressure the compiler has split a value's
+  register there and put the copy (or a reload from scratch) ahead of that
+  instruction, so that the lanes that skipped the branch kept garbage in the
+  new register; as an index it was a wild address.
 
 usage: python3 check_code.py FILE
 """
@@ -97,18 +105,47 @@ def lane_read_hazards(lines):
     return found
 
 
+def early_moves(lines):
+    """(kernel, label, move) of vector moves and reloads ahead of a join's exec."""
+    found = []
+    kernel = label = None
+    moves = None  # since the label, while it may still open a join
+    for text in lines:
+        m = re.match(r"<(\w+)>:$", text)
+        if m:
+            if re.match(r"L\d+$", m[1]):
+                label, moves = m[1], []
+            else:
+                kernel, moves = m[1], None
+            continue
+        if moves is None or not text:
+            continue
+        if re.match(r"s_or_b64 exec, exec, ", text):
+            found += [(kernel, label, t) for t in moves]
+            moves = None
+        elif re.match(r"v_mov_b(32|64)\w* |v_accvgpr_|v_pk_mov_|scratch_load_", text):
+            moves.append(text)
+        elif not re.match(r"s_(?!cbranch|branch|endpgm|setpc|swappc)|v_readlane_|v_writelane_",
+                          text):
+            moves = None  # the block's own work: no join opens here
+    return found
+
+
 def main(argv):
     bad = []
     kernels = 0
     for code in code_objects(argv[1]):
         lines = disassemble(code)
         kernels += sum(1 for t in lines if re.match(r"<_Z\w+>:$", t))
-        bad += lane_read_hazards(lines)
-    for kernel, before, after in bad:
-        print(f"check_code: {kernel}: `{after}` too soon after `{before}`", file=sys.stderr)
+        bad += [f"{k}: `{after}` too soon after `{before}`"
+                for k, before, after in lane_read_hazards(lines)]
+        bad += [f"{k}: `{move}` before the lanes are back at {label}"
+                for k, label, move in early_moves(lines)]
+    for text in bad:
+        print(f"check_code: {text}", file=sys.stderr)
     if bad or not kernels:
         return 1
-    print(f"check_code: {kernels} kernels, lane reads have their wait states")
+    print(f"check_code: {kernels} kernels, lane reads and joins in order")
     return 0
 
 

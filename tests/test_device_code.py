@@ -43,3 +43,26 @@ def test_use_after_lane_read(between, found):
 
 def test_library_lane_reads(listings):
     assert [h for lines in listings for h in check_code.lane_read_hazards(lines)] == []
+
+
+JOIN = "s_or_b64 exec, exec, s[6:7]"
+
+
+@pytest.mark.parametrize("opening,found", [
+    (["v_mov_b32_e32 v26, v126"], 1), (["s_nop 0", "v_mov_b64_e32 v[2:3], v[8:9]"], 1),
+    (["scratch_load_dword v26, off, off offset:16", "s_waitcnt vmcnt(0)"], 1), ([], 0),
+    (["v_readlane_b32 s6, v40, 2", "v_readlane_b32 s7, v40, 3"], 0),
+    (["v_mov_b32_e32 v26, v126", "v_add_u32_e32 v1, v26, v2"], 0),  # the block's own work
+    (["v_mov_b32_e32 v26, v126", "s_cbranch_vccnz L2"], 0),
+])
+def test_move_before_a_join(opening, found):
+    code = ["<_Z1kv>:", "s_and_saveexec_b64 s[6:7], vcc", "s_cbranch_execz L1",
+            "v_mov_b32_e32 v5, v6", "<L1>:", *opening, JOIN, "v_mov_b32_e32 v7, v8"]
+    assert len(check_code.early_moves(code)) == found
+
+
+def test_library_joins(listings):
+    joins = sum(a.startswith("<L") and b.startswith("s_or_b64 exec, exec,")
+                for lines in listings for a, b in zip(lines, lines[1:]))
+    assert joins > 100  # the listings show them as the check expects
+    assert [m for lines in listings for m in check_code.early_moves(lines)] == []
