@@ -99,9 +99,7 @@ struct MgTail
     int off[kMgMaxLevels + 1];
     double* B[kMgMaxLevels];
     double* res[kMgMaxLevels];
-    const MgOp* op;         // of every level
-    const MgTailInfo* info; // level l's cells from info_at[l]
-    int info_at[kMgMaxLevels + 1];
+    int info_at[kMgMaxLevels + 1]; // level l's cells in MgTailTop::info
 };
 
 // What k_mg_tail starts with, by value: the top level's right-hand side and
@@ -110,8 +108,8 @@ struct MgTailTop
 {
     int l0, last, n_top, n_all; // cells of level l0, MgTailInfo in all
     const double* b;
-    const MgTailInfo* info; // MgTail::info
-    const MgOp* op;
+    const MgTailInfo* info; // of the levels from l0 on
+    const MgOp* op;         // of every level
 };
 
 // Which of a level's two vectors k_mg_tail's downward leg leaves the residual

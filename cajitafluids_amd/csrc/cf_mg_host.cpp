@@ -241,7 +241,6 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
         h.last = last;
         h.nu = _nu;
         h.coarse = _coarse;
-        h.op = B.op;
         int off = 0;
         for (int l = 0; l < nl; ++l) {
             h.lev[l] = _lev[l];
@@ -265,7 +264,6 @@ Multigrid::Multigrid(const Geo& g, const cf_config& cfg, hipStream_t s)
         CF_HIP(hipMemcpyAsync(B.info, info.data(), info.size() * sizeof(MgTailInfo),
                               hipMemcpyHostToDevice, s));
         CF_HIP(hipStreamSynchronize(s)); // info is this block's
-        h.info = B.info;
         B.top = MgTailTop{_tail0, last, _lev[_tail0].ncell, (int)info.size(), B.B[_tail0], B.info,
                           B.op};
         CF_HIP(hipMalloc(&p, sizeof(MgTail)));

@@ -1021,8 +1021,7 @@ CoopPlan coop_plan(const Geo& g)
         if (c.strips.G > kCoopMaxGroups)
             return c;
         c.lds = coop_lds(g, c.strips);
-        // window indices fit the slot word's 16 bits
-        if (c.strips.nwin >= (1 << 16) || c.lds > 128 * 1024)
+        if (c.lds > 128 * 1024)
             return c;
         c.groups = c.strips.G;
         c.xch = (size_t)c.groups * (16 + 4 * (size_t)g.n[0]) * sizeof(Word);
