@@ -84,9 +84,13 @@ static void advect_t(const Geo& g, Fields cur, Fields next, hipStream_t s)
 // interpolate's and rk3's, in their order.
 //
 // Bound by vector issue (73% of the cycles at 256^3, 2240 of its ~2700
-// instructions a wave FP64 arithmetic).  Cubic field, against k_advect: 256^3
+// instructions a wave FP64 arithmetic).  The cubic kernel fills the 128
+// registers of four waves a SIMD and spills 25 (56 bytes a lane), the linear
+// one takes 102.  Cubic field, against k_advect: 256^3
 // 2.69 -> 1.87 ms, 190 x 182 x 149 817 -> 590 us, 128^3 338 -> 226, 64^3 64 ->
 // 44; steps of six cells, whose waves mostly gather, 255^3 2.54 -> 2.13 ms.
+// Linear field: 200^3 930 -> 634 us, 64^3 45 -> 33; thin and long grids: 4 x 512
+// x 512 737 -> 608, 512 x 512 x 4 125 -> 103, 8 x 8 x 4096 105 -> 83.
 // Blocks of 1024 with q in the window too: 2.06 ms (one block a CU: nothing
 // runs while it loads).  256 points: one wave less per SIMD.
 //

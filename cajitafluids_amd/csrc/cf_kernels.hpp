@@ -128,7 +128,9 @@ int reduction_blocks_max(const Geo& g);
 // state's stop test or `max_its` iterations of this launch (x, r and the
 // direction p are read at the start and written back at the end, so launches
 // chain).  The same x, r, direction and state bits as the dir_spmv / update
-// pair.
+// pair.  A grid fits with at most 256 strips or pencils of whole x-rows and
+// 4096 cells whose window fits the LDS (2-D: rows of up to 2337 cells) and
+// whose halo is at most 8 cells a lane (3-D: rows of up to 682 cells).
 
 // A 2-D grid's strips: R rows each, G of them; window row pitch e0 = n0 + 2
 // (window index of strip-relative cell (i, jj), halo rows jj = -1 and

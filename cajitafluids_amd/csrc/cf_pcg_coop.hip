@@ -77,7 +77,10 @@ constexpr unsigned kCoopSpin = 1u << 22; // polls (about 1 us each) before a wai
 // 700 x 500 -, 14.9, 10.5; 1024^2 -, -, 16.9.  Now, at the shape chosen: 32^2
 // 2.0, 128^2 4.3, 256^2 5.6, 391 x 263 6.2, 512^2 7.1, 700 x 500 9.0, 1024^2
 // 14.7 (the streaming kernels 32.2).  1024 lanes, and 2 cells a lane, were
-// slower or within 2% everywhere.
+// slower or within 2% everywhere.  Rows of more than 1024 cells, whose halo is
+// as large as the strip, gain too (300 iterations, over them, the kernels
+// before and these): 1100 x 200 21.1, 9.8; 1700 x 250 29.1, 12.2; 2300 x 256
+// 33.8, 21.2; 2300 x 30 32.5, 12.8.
 CoopGrid coop_grid(const Geo& g)
 {
     constexpr int shape[3][3] = {{256, 4, 64}, {512, 4, 128}, {448, 10, kCoopMaxGroups}};

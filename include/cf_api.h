@@ -230,9 +230,10 @@ cf_status cf_set_kernel_timing(cf_solver* h, int enable);
 /* kernel: 0 FP64 direction+SpMV, 1 FP64 update, 2 FP64 finalize kernels
  * (unused), 3-5 the same for the FP32 inner solve, 6 advection, 7 FP64
  * defect-correction residual, 8 one multigrid V-cycle (all its kernels),
- * 9 one launch of the cooperative PCG that 2-D and small 3-D grids (up to
- * 256 strips or pencils of whole rows and 4096 cells) run in place of 0 and
- * 1, the 3-D ones also in place of 3 and 4 */
+ * 9 one launch of the cooperative PCG, which runs in place of 0 and 1 on 2-D
+ * grids of up to 256 strips of whole rows and 4096 cells (rows of up to 2337
+ * cells), and in place of 0, 1, 3 and 4 on 3-D grids of up to 256 pencils of
+ * whole x-rows and 4096 cells (rows of up to 682 cells; about 100^3) */
 cf_status cf_kernel_time(cf_solver* h, int kernel, double* total_ms,
                          int64_t* launches);
 cf_status cf_reset_kernel_time(cf_solver* h);
